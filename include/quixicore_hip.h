@@ -98,7 +98,7 @@ int qc_hip_qgemm(int format, const void* packed, const float* x, float* y, long 
  * are safe (their launch sequences queue one after the other); calls on
  * different streams of one GPU can overlap on the device and race: serialize
  * those.  M >= 2 runs passes of at
- * most 32 rows (never the 2-D M >= 64 route, whose scratch grows with m) with
+ * most 32 rows (never the 2-D route, whose scratch grows with m) with
  * the fewest K splits.  Limits: m <= QC_QGEMM_NOALLOC_MAX_M and
  * k <= QC_QGEMM_NOALLOC_MAX_K, else 1 (QC_INVALID_SHAPE) with a message in
  * qc_hip_last_error().  Within k <= 8192 every such call fits; above it, a
@@ -359,7 +359,7 @@ int qc_hip_set_int8_gemm_route(int route);
 int qc_hip_set_qgemm_plan(int waves, int stages);
 
 /* Route of qc_hip_qgemm for M >= 2 (K % 64 == 0): 0 (the default) runs the
- * 2-D tiled GEMM for M >= 64 and passes of at most 32 rows below; -1 always
+ * 2-D tiled GEMM for M >= 33 and one pass of at most 32 rows below; -1 always
  * uses the passes; 1 / 2 always use the 2-D GEMM with one / two K ranges.
  * Results stay within the contract tolerance on every route.  Tuning and
  * test knob with no reference counterpart. */

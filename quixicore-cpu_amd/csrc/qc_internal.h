@@ -42,7 +42,7 @@ struct GemvTuning {
   int rows_per_wave = 0;  // GEMV rows per wavefront (1, 2, 4, 7, 8, 14; 0 = from the shape)
   int qgemm_waves = 0;    // small-batch GEMM waves per workgroup (4, 8; 0 = from the shape)
   int qgemm_stages = 0;   // small-batch GEMM K stages per workgroup (1..16; 0 = from the shape)
-  int qgemm_panel = 0;    // 2-D GEMM route: 0 = for m >= 64, -1 = never, 1 / 2 = always (K ranges)
+  int qgemm_panel = 0;    // 2-D GEMM route: 0 = for m >= 33, -1 = never, 1 / 2 = always (K ranges)
   int qgemm_rows = 0;     // exact-digit rows route for 2 <= m <= 8: 0 = by shape, -1 = never, 1 = always
   int qgemm_fold = 0;     // digit-layout GEMM builds its own digits: 0 = where it can, -1 = never
   int cint8_dot = 0;      // canonical int8, M = 1: digit-dot kernel 0 = where it applies, -1 = never
@@ -95,14 +95,20 @@ hipError_t launch_qgemv_w8a8(int fmt, const void* W, const float* x, float* y, l
                              long long k, int rows_per_wave, int* status, hipStream_t s);
 
 // GEMM on MFMA (m >= 2, K % 64 == 0, W 4-byte aligned): int8 digit planes
-// for up to 8 rows per pass, bf16 hi/lo above; for m >= 64 one 2-D tiled
-// kernel (the panel route) instead of passes of 32 rows.  waves / stages:
+// for up to 8 rows per pass, f16 / bf16 hi/lo above; from 33 rows one 2-D
+// tiled GEMM (launch_qgemm_wide) instead of passes of 32 rows.  waves / stages:
 // small-batch plan override (0 = from the shape); panel: 0 = from m, -1 =
 // never, 1 / 2 = always (one / two K ranges).  fold: 0 = the digit-layout
 // GEMM builds its own digits where it can (no prep launch), -1 = never.
 hipError_t launch_qgemm_mfma(int fmt, const void* W, const float* x, float* y, int m, int n,
                              int k, hipStream_t s, int waves = 0, int stages = 0,
                              int panel = 0, int fold = 0);
+
+// The 2-D tiled route of launch_qgemm_mfma (m >= 2, K % 64 == 0, W 4-byte
+// aligned): f16 MFMA over hi / lo activations.  ranges: K ranges, 0 = from
+// the shape.  The caller holds ws->call.
+hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, int m, int n,
+                             int k, int ranges, hipStream_t s, StreamWorkspace* ws);
 
 // launch_qgemm_mfma without allocating: the scratch is a fixed device
 // array of kQgemmNoAllocScratchBytes per GPU, shared by every such call on

@@ -1,6 +1,7 @@
 // Small-batch q8_0 / q4_0 GEMM (2 <= M, in tiles of 16 activation rows) on
 // gfx950 MFMA: int8 digit planes for up to 8 rows per pass, f16 (q8_0) or
-// bf16 (q4_0) operands above, and a 2-D tiled kernel for M >= 64.
+// bf16 (q4_0) operands above.  From 33 rows a call takes the 2-D tiled GEMM
+// (qgemm_wide.hip) instead of passes of 32.
 //
 // Semantics as the reference's qgemm (kernels/quantization/qgemm_ref.cpp:
 // 156-162, one qgemv per activation row: y[m][n] = sum_b d[n][b] *
@@ -199,7 +200,7 @@ __device__ __forceinline__ void ring_barrier() {
 // of v - hi (bytes 1024..2047), and (q4_0) the bias -8 * sum(hi + lo) per
 // row and block, the MFMA's C input for the nibble offset.  Small-batch
 // passes store fragment (b, t) at b * T + t over nbp blocks (those past K
-// zero), the panel route at t * nb + b.
+// zero).
 //
 // Per-row power-of-two scale: the fragments hold v = x * 2^-e(m), with e(m)
 // from the frexp exponent of max |x[m][:]| (0 for a zero or non-finite row)
@@ -240,7 +241,7 @@ inline int clear_workgroups(long long count) {
   return static_cast<int>(w < 512 ? w : 512);
 }
 
-template <bool PANEL, bool BIAS>
+template <bool BIAS>
 __global__ __launch_bounds__(256) void prep_rows(const float* __restrict__ x, int M, int K,
                                                  int nbo, int T, uint8_t* __restrict__ xf,
                                                  float* __restrict__ bias,
@@ -348,8 +349,7 @@ __global__ __launch_bounds__(256) void prep_rows(const float* __restrict__ x, in
       for (int i = 0; i < 16; ++i) v[i] = 0.0f;
     }
     float sc[2];
-    const long long f = PANEL ? static_cast<long long>(t) * nbo + blk
-                              : static_cast<long long>(blk) * T + t;
+    const long long f = static_cast<long long>(blk) * T + t;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       using Op = std::conditional_t<BIAS, bf16x8, f16x8>;
@@ -1142,7 +1142,7 @@ hipError_t run(const uint8_t* W, const float* x, float* y, int m, int n, int k, 
                                                                tail_src, tail, tail_pad,
                                                                static_cast<int>(pad_bytes));
     else
-      prep_rows<false, FMT == kQ4_0>
+      prep_rows<FMT == kQ4_0>
           <<<XL + (ks == 2 ? clear_workgroups(outs) : 0), 256, 0, s>>>(
               x, m, k, nbp, XB::T, xf, bias, rexp, y, ks == 2 ? outs : 0, tail_src, tail,
               tail_pad, static_cast<int>(pad_bytes), XL);
@@ -1174,339 +1174,6 @@ hipError_t run(const uint8_t* W, const float* x, float* y, int m, int n, int k, 
   return hipGetLastError();
 }
 
-// ------------------------------------------------ panel route, M >= 64 ---
-//
-// The reference switches qgemm_prepacked to a row-panel GEMM at M >= 64
-// (kernels/quantization/qgemm_panel.cpp:234-286).  Here every M >= 64 call
-// (qgemm and qgemm_prepacked) runs one 2-D tiled GEMM instead of passes of 32
-// rows, each of which re-streams the whole weight matrix.  Numerics are those
-// of the f16 / bf16 passes above (hi/lo activations, exact codes, per-block
-// f32 scaling), so the contract bound is unchanged.
-//
-// Workgroup: 8 wavefronts as 2 (m) x 4 (n), each computing 64 x 64 outputs
-// as 4 x 4 tiles of v_mfma_f32_16x16x32_{f16,bf16}; workgroup tile 128 x 256.  K
-// runs in stages of one block pair (64 elements) through a 3-deep LDS ring
-// filled by global_load_lds: the activation fragments of the workgroup's 8
-// m-tiles (hi, lo, and the q4_0 bias) as 16-byte chunks, and the pair's bytes
-// of its 256 weight rows as dwords.  Every wavefront issues the same loads
-// per stage (spare weight lanes re-read a valid dword into padding), so the
-// waits are exact counts, as in the small-batch kernel.
-constexpr int kPTN = 4;                           // 16x16 tiles per wave (n)
-constexpr int kPWM = 2, kPWN = 4;                 // waves per workgroup (m, n)
-constexpr int kPWaves = kPWM * kPWN;
-constexpr int kPBN = 16 * kPTN * kPWN;            // 256 rows of W per workgroup
-
-// TM: 16x16 tiles per wave along m (4: 128 x 256 workgroup tiles with a
-// 3-deep ring; 8: 256 x 256 with a 2-deep ring).
-template <int FMT, int TM>
-struct PanelStage {
-  static constexpr bool bias = FMT == kQ4_0;
-  static constexpr int bm = 16 * TM * kPWM;                         // rows of x per workgroup
-  static constexpr int mt = bm / 16;                                // m-tiles per workgroup
-  static constexpr int pd = PairLayout<FMT>::bytes / 4;             // 17 / 9 dwords per row
-  static constexpr int x_bytes = mt * 2 * kFragBytes;               // 32 / 64 KB
-  static constexpr int x_loads = x_bytes / 16 / (64 * kPWaves);     // 4 / 8 chunks per lane
-  static constexpr int b_bytes = bias ? mt * 2 * 64 : 0;            // 1 / 2 KB
-  static constexpr int w_dwords = kPBN * pd;
-  static constexpr int w_loads = (w_dwords + 64 * kPWaves - 1) / (64 * kPWaves);  // 9 / 5
-  static constexpr int w_bytes = kPWaves * w_loads * 256;           // with padding
-  static constexpr int bytes = x_bytes + b_bytes + w_bytes;
-  static constexpr int ring = 3 * bytes <= 160 * 1024 ? 3 : 2;
-  static constexpr int g = x_loads + (bias ? 1 : 0) + w_loads;      // loads per wave per stage
-  static_assert(x_bytes % (16 * 64 * kPWaves) == 0, "whole x loads");
-  static_assert(ring * bytes <= 160 * 1024, "LDS");
-  static_assert(g * (ring - 1) < 64, "vmcnt range");
-  static_assert(mt % kPWaves == 0 && mt / kPWaves <= 8 && ((mt / kPWaves) & (mt / kPWaves - 1)) == 0,
-                "bias loads: 8 lanes per m-tile, a power-of-two count of whole m-tiles per wave");
-};
-
-template <int FMT, int TM>
-__global__ __launch_bounds__(64 * kPWaves, 1) void qgemm_panel(
-    const uint8_t* __restrict__ W, const uint8_t* __restrict__ xf, const float* __restrict__ bias,
-    float* __restrict__ y, const int* __restrict__ rexp, const float* __restrict__ x, int M,
-    int N, int K, int pairs_per_split, int ks_count) {
-  using PS = PanelStage<FMT, TM>;
-  constexpr int PB = PairLayout<FMT>::bytes;
-  constexpr int G = PS::g;
-  constexpr int R = PS::ring;
-  constexpr int BR = PS::mt / kPWaves;           // bias m-tiles per wave (1 / 2)
-  __shared__ __attribute__((aligned(1024))) uint8_t ring0[PS::bytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t ring1[PS::bytes];
-  __shared__ __attribute__((aligned(1024))) uint8_t ring2[R > 2 ? PS::bytes : 16];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % kPWM, wn = wave / kPWM;
-  const int j = lane >> 4;
-  const int n0 = blockIdx.x * kPBN;
-  const int mt0 = blockIdx.y * PS::mt;
-  const int nb = K / 32, npairs = K / 64;
-  const int p0 = blockIdx.z * pairs_per_split;
-  const int p1 = min(p0 + pairs_per_split, npairs);
-  const long long row_bytes = static_cast<long long>(nb) * (PB / 2);
-
-  // Sources: a wave-uniform base per workgroup and stage (scalar registers)
-  // plus a per-lane 32-bit offset that never changes, so issuing a stage
-  // costs no vector arithmetic.  x chunk c = (wave * x_loads + i) * 64 + lane:
-  // m-tile c >> 8, byte 16 (c & 255) of its pair (blocks 2p, 2p + 1 adjacent).
-  const uint8_t* xbase = xf + static_cast<long long>(mt0) * nb * kFragBytes;
-  uint32_t xoff[PS::x_loads];
-#pragma unroll
-  for (int i = 0; i < PS::x_loads; ++i) {
-    const int c = (wave * PS::x_loads + i) * 64 + lane;
-    xoff[i] = static_cast<uint32_t>((c >> 8) * nb * kFragBytes + 16 * (c & 255));
-  }
-  // bias: wave w, lanes 0 .. 8 BR - 1, 128 B of each of m-tiles
-  // BR w .. BR w + BR - 1 (the pair's two blocks)
-  const uint8_t* bbase = reinterpret_cast<const uint8_t*>(bias) +
-                         static_cast<long long>(mt0) * nb * 64;
-  const uint32_t boff = static_cast<uint32_t>((wave * BR + ((lane >> 3) & (BR - 1))) * nb * 64 +
-                                              16 * (lane & 7));
-  // weight dword d = (wave * w_loads + i) * 64 + lane: row d / pd, dword
-  // d % pd; d past the stage re-reads the stage's last dword
-  const uint8_t* wbase = W + static_cast<long long>(n0) * row_bytes;
-  uint32_t woff[PS::w_loads];
-#pragma unroll
-  for (int i = 0; i < PS::w_loads; ++i) {
-    int d = (wave * PS::w_loads + i) * 64 + lane;
-    d = d < PS::w_dwords ? d : PS::w_dwords - 1;
-    const int r = min(n0 + d / PS::pd, N - 1) - n0;
-    woff[i] = static_cast<uint32_t>(r * row_bytes + 4 * (d % PS::pd));
-  }
-  auto slot_base = [&](int slot) -> uint8_t* { return slot == 0 ? ring0 : slot == 1 ? ring1 : ring2; };
-  // Load l (0 .. G - 1; a constant after unrolling) of stage p into a slot:
-  // the x chunks, then (q4_0) the bias, then the weight dwords.
-  auto issue_one = [&](int p, int slot, int l) {
-    uint8_t* base = slot_base(slot);
-    if (l < PS::x_loads) {
-      dma16(xbase + static_cast<long long>(2 * p) * kFragBytes, xoff[l < PS::x_loads ? l : 0],
-            base + 16 * (wave * PS::x_loads + l) * 64);
-    } else if (PS::bias && l == PS::x_loads) {
-      if (lane < 8 * BR) dma16(bbase + 128 * p, boff, base + PS::x_bytes + 128 * BR * wave);
-    } else {
-      const int wl = l - PS::x_loads - (PS::bias ? 1 : 0);
-      dma4(wbase + static_cast<long long>(p) * PB, woff[wl >= 0 ? wl : 0],
-           base + PS::x_bytes + PS::b_bytes + 256 * (wave * PS::w_loads + wl));
-    }
-  };
-  auto issue = [&](int p, int slot) {
-#pragma unroll
-    for (int l = 0; l < G; ++l) issue_one(p, slot, l);
-  };
-
-  f32x4 acc[TM][kPTN];
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < kPTN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // Decoded weight fragments of one half stage (one block of the pair):
-  // codes as bf16 and the block scales of the wave's 4 n-tiles.
-  using Op = typename OpType<FMT>::T;
-  struct HalfW {
-    Op w[kPTN];
-    float d[kPTN];
-  };
-  auto decode = [&](int slot, int h, HalfW& o) {
-    const uint32_t* sw = reinterpret_cast<const uint32_t*>(slot_base(slot) + PS::x_bytes + PS::b_bytes);
-#pragma unroll
-    for (int tn = 0; tn < kPTN; ++tn) {
-      const uint32_t* pr = sw + (wn * 64 + tn * 16 + (lane & 15)) * PS::pd;
-      uint32_t c0, c1, dbits;
-      if (h == 0) {
-        const uint32_t b0x = pr[PairLayout<FMT>::blk0_dword(j)];
-        const uint32_t b0y = pr[PairLayout<FMT>::blk0_dword(j) + 1];
-        const uint32_t b0z = pr[PairLayout<FMT>::blk0_dword(j) + 2];
-        c0 = __builtin_amdgcn_alignbyte(b0y, b0x, 2);
-        c1 = __builtin_amdgcn_alignbyte(b0z, b0y, 2);
-        dbits = pr[0] & 0xFFFFu;
-      } else {
-        c0 = pr[PairLayout<FMT>::blk1_dword(j)];
-        c1 = pr[PairLayout<FMT>::blk1_dword(j) + 1];
-        dbits = pr[PairLayout<FMT>::scale1_dword] >> 16;
-      }
-      o.w[tn] = codes_op<FMT>(c0, c1, j);
-      o.d[tn] = half_bits_to_float(dbits);
-    }
-  };
-  // The 2 x kPTN MFMAs of m-tile tm against one decoded half, each tile's
-  // block sum scaled into the accumulators.
-  auto mma = [&](int slot, int h, int tm, const HalfW& hw) {
-    const uint8_t* base = slot_base(slot);
-    const int mt = wm * TM + tm;
-    const uint8_t* f = base + (mt * 2 + h) * kFragBytes + 16 * lane;
-    const Op xh = *reinterpret_cast<const Op*>(f);
-    const Op xl = *reinterpret_cast<const Op*>(f + 1024);
-    f32x4 c0 = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (PS::bias)
-      c0 = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(base + PS::x_bytes) +
-                                           (mt * 2 + h) * 16 + 4 * j);
-#pragma unroll
-    for (int tn = 0; tn < kPTN; ++tn) {
-      f32x4 c = mfma_op(xh, hw.w[tn], c0);
-      c = mfma_op(xl, hw.w[tn], c);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[tm][tn][e] = fmaf(c[e], hw.d[tn], acc[tm][tn][e]);
-    }
-  };
-  auto pin_acc = [&]() {
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-#pragma unroll
-      for (int b = 0; b < kPTN; ++b) asm volatile("" : "+v"(acc[a][b]));
-  };
-
-  // Ring of R stages.  Stages p0 .. p0 + R - 2 are in flight before the
-  // loop.  Step i starts with the wave's wait for stage p0 + i + 1 and a
-  // workgroup barrier, after which that stage is visible to every wave and
-  // no wave reads stage p0 + i - 1, whose slot receives stage p0 + i + R - 1.
-  // Those loads are spread over block 0's MFMAs so that the eight waves do
-  // not queue them all at once.  Weights are decoded one half stage ahead:
-  // block 1's decode overlaps block 0's MFMAs, and block 0 of stage
-  // p0 + i + 1 is decoded during block 1's.  Past the last stage the loads
-  // repeat stage p1 - 1 into the free slot and the decode reads a slot whose
-  // result is unused, so every step is the same straight-line code.
-  // Unrolled by the ring depth so every slot index is a constant.
-  static_assert(R >= 3, "the next stage must land while the current one is read");
-  const int count = p1 - p0;
-  if (count > 0) {
-#pragma unroll
-    for (int i = 0; i < R - 1; ++i)
-      if (i < count) issue(p0 + i, i);
-    wait_stages<G, R - 2>(min(R - 2, count - 1));
-    wait_lgkmcnt0();
-    ring_barrier();
-    HalfW h0, h1;
-    decode(0, 0, h0);
-    auto step = [&](int i, int slot) {
-      // stages issued after stage i + 1 and possibly still in flight
-      wait_stages<G, R - 3>(min(R - 3, count - 2 - i));
-      wait_lgkmcnt0();
-      ring_barrier();
-      const int pi = min(p0 + i + R - 1, p1 - 1);
-      const int si = (slot + R - 1) % R;
-      decode(slot, 1, h1);
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-#pragma unroll
-        for (int l = tm * G / TM; l < (tm + 1) * G / TM; ++l) issue_one(pi, si, l);
-        mma(slot, 0, tm, h0);
-      }
-      decode((slot + 1) % R, 0, h0);
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) mma(slot, 1, tm, h1);
-      pin_acc();
-    };
-    for (int i = 0; i < count; i += R) {
-#pragma unroll
-      for (int u = 0; u < R; ++u)
-        if (i + u < count) step(i + u, u);
-    }
-  }
-  wait_vmcnt<0>();   // no global->LDS load may outlive the workgroup's LDS
-
-  // acc[tm][tn][e] is output (m = 16 (mt0 + 4 wm + tm) + 4 j + e,
-  // n = n0 + 64 wn + 16 tn + (lane & 15)).
-  bool special = false;
-#pragma unroll
-  for (int tn = 0; tn < kPTN; ++tn) {
-    const int n = n0 + wn * 64 + tn * 16 + (lane & 15);
-    if (n >= N) continue;
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = 16 * (mt0 + wm * TM + tm) + 4 * j + e;
-        if (m >= M) continue;
-        const long long o = static_cast<long long>(m) * N + n;
-        const int r = rexp[m];
-        if (r == kRowNonfinite) {   // stored by the loop below
-          special = true;
-          continue;
-        }
-        const float v = ldexpf(acc[tm][tn][e], r);   // undo the row scale
-        if (ks_count == 1) y[o] = v;
-        else atomicAdd(y + o, v);
-      }
-    }
-  }
-  // Rows holding NaN or +-inf: the reference's f32 form over this K range.
-  if (__any(special)) {
-#pragma unroll 1
-    for (int q = 0; q < kPTN * TM * 4; ++q) {
-      const int tn = q / (TM * 4), tm = (q / 4) % TM, e = q % 4;
-      const int n = n0 + wn * 64 + tn * 16 + (lane & 15);
-      const int m = 16 * (mt0 + wm * TM + tm) + 4 * j + e;
-      if (n >= N || m >= M || rexp[m] != kRowNonfinite) continue;
-      const float v = nonfinite_blocks_f32<FMT>(W + static_cast<long long>(n) * row_bytes,
-                                                x + static_cast<long long>(m) * K, 2 * p0, 2 * p1);
-      const long long o = static_cast<long long>(m) * N + n;
-      if (ks_count == 1) y[o] = v;
-      else atomicAdd(y + o, v);
-    }
-  }
-}
-
-// K ranges of the 2-D GEMM: two (atomic adds onto a cleared y, two addends
-// onto zero: order-independent) when both halves' workgroups still run in one
-// round at one workgroup per CU, else one.
-int panel_split(int m, int n, int k, int cus, int bm) {
-  const long long tiles = static_cast<long long>((m + bm - 1) / bm) * ((n + kPBN - 1) / kPBN);
-  return 2 * tiles <= cus && k / 64 >= 2 ? 2 : 1;
-}
-
-// Route for m >= 64 from two time models fitted on MI355X (q8_0 and q4_0
-// alike): a 2-D GEMM workgroup spends ~2.45 us per block pair of its K range
-// (MFMA and VALU issue bound, independent of how full the chip is), in
-// ceil(workgroups / CUs) rounds; a pass of 32 rows costs max(N K / 2.3e12 s,
-// 17 us).  The passes win for small M at small N or long K.
-bool panel_pays(int m, int n, int k, int cus) {
-  constexpr int bm = PanelStage<kQ8_0, 4>::bm;
-  const int ks = panel_split(m, n, k, cus, bm);
-  const long long tiles = static_cast<long long>((m + bm - 1) / bm) * ((n + kPBN - 1) / kPBN);
-  const long long rounds = (tiles * ks + cus - 1) / cus;
-  const double panel = rounds * ((k / 64 + ks - 1) / ks) * 2.45e-6 + 4e-6;
-  const double passes = ((m + 31) / 32) * std::max(static_cast<double>(n) * k / 2.3e12, 17e-6);
-  return panel < passes;
-}
-
-template <int FMT, int TM>
-hipError_t run_panel(const uint8_t* W, const float* x, float* y, int m, int n, int k,
-                     hipStream_t s, int split, int* rexp, Scratch& scratch) {
-  using PS = PanelStage<FMT, TM>;
-  if (rexp == nullptr) return hipErrorInvalidValue;   // per-row exponents (see prep_rows)
-  const int nb = k / 32, npairs = k / 64;
-  const int mblocks = (m + PS::bm - 1) / PS::bm, nblocks = (n + kPBN - 1) / kPBN;
-  const int mtiles = mblocks * PS::mt;
-  // per-lane 32-bit source offsets within a workgroup's rows
-  if (static_cast<long long>(kPBN) * nb * (PairLayout<FMT>::bytes / 2) >= (1LL << 32) ||
-      static_cast<long long>(PS::mt) * nb * kFragBytes >= (1LL << 32))
-    return hipErrorInvalidValue;
-  int ks = panel_split(m, n, k, device_cu_count(), PS::bm);
-  if (split == 1 || split == 2) ks = split;
-  if (npairs < 2) ks = 1;
-  const int per = (npairs + ks - 1) / ks;
-  const size_t xf_bytes = static_cast<size_t>(mtiles) * nb * kFragBytes;
-  const size_t bias_bytes = FMT == kQ4_0 ? static_cast<size_t>(mtiles) * nb * 64 : 0;
-  void* ws = nullptr;
-  hipError_t e = scratch.get(s, xf_bytes + bias_bytes + 256, &ws);
-  if (e != hipSuccess) return e;
-  uint8_t* xf = static_cast<uint8_t*>(ws);
-  float* bias = reinterpret_cast<float*>(xf + xf_bytes);
-  const long long outs = static_cast<long long>(m) * n;
-  prep_rows<true, FMT == kQ4_0>
-      <<<static_cast<unsigned>(16 * mtiles + (ks == 2 ? clear_workgroups(outs) : 0)), 256, 0, s>>>(
-          x, m, k, nb, 0, xf, bias, rexp, y, ks == 2 ? outs : 0, nullptr, 0, nullptr, 0,
-          16 * mtiles);
-  e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const dim3 grid(static_cast<unsigned>(nblocks), static_cast<unsigned>(mblocks),
-                  static_cast<unsigned>(ks));
-  qgemm_panel<FMT, TM><<<grid, 64 * kPWaves, 0, s>>>(W, xf, bias, y, rexp, x, m, n, k, per, ks);
-  return hipGetLastError();
-}
-
 }  // namespace
 
 namespace {
@@ -1514,21 +1181,21 @@ namespace {
 hipError_t qgemm_mfma_with(int fmt, const void* W, const float* x, float* y, int m, int n, int k,
                            hipStream_t s, int waves, int stages, int panel, Scratch& scratch) {
   const auto* w = static_cast<const uint8_t*>(W);
-  // panel: 0 = from the shape (for m >= 64), -1 = never, 1 / 2 = always
-  // (for m >= 2) with one / two K ranges
-  const bool use_panel = panel > 0 || (panel == 0 && m >= 64 && panel_pays(m, n, k, device_cu_count()));
-  // The bf16 layouts (the panel and passes of more than 8 rows) scale each
-  // row by its power of two; their prep kernels store the exponents here.
+  // panel: 0 = from m, -1 = never, 1 / 2 = always (for m >= 2) with one / two
+  // K ranges.  From 33 rows a pass of 32 would stream the weights twice.  A
+  // forced small-batch plan keeps the passes below 64 rows.
+  const bool forced = waves != 0 || stages != 0;
+  if (scratch.w != nullptr && (panel > 0 || (panel == 0 && m > (forced ? 63 : 32))))
+    return launch_qgemm_wide(fmt, W, x, y, m, n, k, panel, s, scratch.w);
+  // The f16 / bf16 layouts (passes of more than 8 rows) scale each row by its
+  // power of two; their prep kernel stores the exponents here.
   int* rexp = nullptr;
-  if (use_panel || m > 8) {
+  if (m > 8) {
     void* p = nullptr;
     hipError_t e = scratch.get(s, sizeof(int) * static_cast<size_t>(m) + 256, &p, 1);
     if (e != hipSuccess) return e;
     rexp = static_cast<int*>(p);
   }
-  if (use_panel)
-    return fmt == kQ8_0 ? run_panel<kQ8_0, 4>(w, x, y, m, n, k, s, panel, rexp, scratch)
-                        : run_panel<kQ4_0, 4>(w, x, y, m, n, k, s, panel, rexp, scratch);
   for (int m0 = 0; m0 < m; m0 += 32) {
     const int mt = m - m0 < 32 ? m - m0 : 32;
     const float* xm = x + static_cast<long long>(m0) * k;
@@ -1617,7 +1284,7 @@ hipError_t launch_qgemm_mfma_noalloc(int fmt, const void* W, const float* x, flo
   scratch.max_ks = 2;
   if (scratch.fixed_split >= scratch.fixed_bytes) return hipErrorOutOfMemory;
   std::lock_guard<std::mutex> hold(d->call);   // until the call's last launch
-  // passes of at most 32 rows: the panel route's fragments grow with m
+  // passes of at most 32 rows: the 2-D route's fragments grow with m
   return qgemm_mfma_with(fmt, W, x, y, m, n, k, s, 0, 0, -1, scratch);
 }
 

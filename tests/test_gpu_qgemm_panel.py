@@ -94,3 +94,35 @@ def test_panel_prefill_sizes(qc, oracle, dev, fmt, m, n, k):
     x = torch.randn((m, k), generator=g, device=dev).cpu().numpy()
     y = _run(qc, dev, fmt, P, x, n, k, 0)
     _check(oracle, fmt, P.cpu().numpy(), x, y, n, k, (0, 1, m // 2, m - 1))
+
+
+# Automatic route: 33 rows is the first 2-D call, and shapes around the edges
+# of its tiles (64 / 128 / 256 rows by 128 / 256 columns), with K of one block
+# pair, odd pairs, and K splits; from 384 rows and 2048 columns q4_0 takes the
+# re-encoded 6-bit form.
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(33, 129, 64), (64, 2048, 4096), (65, 127, 320),
+                                   (77, 1361, 1088), (257, 300, 448), (383, 2049, 192),
+                                   (384, 2048, 64), (385, 2079, 576), (641, 2305, 128),
+                                   (1025, 4097, 192), (2049, 2080, 64)])
+def test_wide_tile_edges(qc, oracle, dev, fmt, m, n, k):
+    import torch
+    print(f"wide fmt={fmt} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    P = qc.pack(fmt, torch.randn((n, k), generator=g, device=dev) * 0.02)
+    x = torch.randn((m, k), generator=g, device=dev)
+    x[torch.rand((m, k), generator=g, device=dev) < 0.01] *= 20.0
+    Y = [torch.full((m, n), float("nan"), device=dev) for _ in range(2)]
+    for y in Y:
+        assert qc.qgemm_raw(fmt, P, x, y, m, n, k) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(Y[0].view(torch.int32), Y[1].view(torch.int32))
+    w = torch.from_numpy(oracle.unpack(fmt, P.cpu().numpy(), n, k)).to(dev).double()
+    y64 = x.double() @ w.T.contiguous()
+    bound = TOL * x.double().norm(dim=1, keepdim=True) * w.norm(dim=1)[None, :]
+    err = (Y[0].double() - y64).abs()
+    assert bool((err <= bound).all()), float((err / bound).max()) * TOL
+    # as a whole the result is far closer than one output's bound: the f16 pair
+    # keeps 2^-22 of each element
+    rel = float((Y[0].double() - y64).norm() / y64.norm())
+    assert rel < 1e-6, rel
