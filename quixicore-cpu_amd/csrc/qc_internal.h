@@ -110,6 +110,12 @@ hipError_t launch_qgemm_mfma(int fmt, const void* W, const float* x, float* y, i
 hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, int m, int n,
                              int k, int ranges, hipStream_t s, StreamWorkspace* ws);
 
+// The q4_0 form of it that re-encodes weights and activations for the
+// block-scaled 6-bit MFMA, and the sizes it is taken for.
+bool mx_pays(int m, int n);
+hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n, int k,
+                           hipStream_t s, StreamWorkspace* ws);
+
 // launch_qgemm_mfma without allocating: the scratch is a fixed device
 // array of kQgemmNoAllocScratchBytes per GPU, shared by every such call on
 // that GPU (calls must not overlap).  Passes of at most 32 rows, the fewest

@@ -1,4 +1,5 @@
-// Pieces of the 2-D tiled q8_0 / q4_0 GEMM (qgemm_wide.hip): grids of 32 x 32 MFMA tiles per wave, operands streamed
+// Pieces shared by the 2-D tiled q8_0 / q4_0 GEMMs (qgemm_wide.hip,
+// qgemm_mx.hip): grids of 32 x 32 MFMA tiles per wave, operands streamed
 // through an LDS ring with explicit waits.
 #pragma once
 

@@ -1,7 +1,7 @@
 // Small-batch q8_0 / q4_0 GEMM (2 <= M, in tiles of 16 activation rows) on
 // gfx950 MFMA: int8 digit planes for up to 8 rows per pass, f16 (q8_0) or
-// bf16 (q4_0) operands above.  From 33 rows a call takes the 2-D tiled GEMM
-// (qgemm_wide.hip) instead of passes of 32.
+// bf16 (q4_0) operands above.  From 33 rows a call takes the 2-D tiled GEMMs
+// (qgemm_wide.hip, qgemm_mx.hip) instead of passes of 32.
 //
 // Semantics as the reference's qgemm (kernels/quantization/qgemm_ref.cpp:
 // 156-162, one qgemv per activation row: y[m][n] = sum_b d[n][b] *
