@@ -856,6 +856,24 @@ hipError_t launch_cint8(const CInt8Launch& L, hipStream_t s) {
   bool fast = k % 16 == 0 && (!grp || (sg.gsize >= 16 && (1 << sg.gshift) == sg.gsize));
   for (int i = 0; i < L.nw; ++i)
     fast = fast && reinterpret_cast<uintptr_t>(L.w[i].codes) % 16 == 0;
+  // From some tens of rows: f16 MFMA where it measured faster than the row
+  // planes (K = 4096, us, planes / f16 with 16-bit and f32 activations).  Groups
+  // of 32, from 33 rows: N = 4096 M = 33 101 / 50, M = 128 150 / 53; N = 14336
+  // M = 512 586 / 151.  Other groups, from 65 rows: groups of 128 N = 4096 M =
+  // 64 43 / 46 and 52, M = 128 67 / 46 and 54; N = 14336 M = 128 75 / 59 and
+  // 64, M = 512 257 / 120 and 155.  Row scales from 129 rows while the planes'
+  // 64 x 256 output tiles fill at most half of the CUs: N = 4096 M = 256 60 /
+  // 37 and 47, M = 512 63 / 41 and 54; N = 14336 M = 256 67 / 70 and 95.  (Every
+  // rule is the same for f32 and 16-bit activations, whose results have the
+  // same bits.)  Lengths the planes do not take go here as well.
+  const long long plane_tiles = (m + 63LL) / 64 * ((L.w[0].rows * (L.mode == 1 ? 2 : 1) + 255) / 256);
+  const bool planes_fit = k <= kPlanesMaxK && (!grp || k % 128 == 0);
+  const bool f16_pays = !grp              ? m > 128 && 2 * plane_tiles <= device_cu_count()
+                        : sg.gsize == 32 ? m > 32
+                                         : m > 64;
+  if (fast && L.dot == 0 && L.mode != 2 && k % 64 == 0 &&
+      (!grp || sg.gsize == 32 || sg.gsize % 64 == 0) && (f16_pays || (!planes_fit && m > 32)))
+    return launch_cint8_f16(sg, L, m, k, s);
   // Two or more activation rows with row scales, three or more with scale
   // groups of 64 or a multiple of 128 columns, five or more with groups of
   // 32: the digit planes on the int8 MFMA GEMM (the row-plane route,

@@ -1,6 +1,7 @@
 // Shared by the canonical int8 projection kernels: canonical_int8.hip (the
 // digit-dot, f32 multiply-add and generic kernels, and the routing) and
-// canonical_planes.hip (the row-plane route on the int8 MFMA GEMM).
+// canonical_planes.hip (the row-plane route on the int8 MFMA GEMM) and
+// canonical_f16.hip (the f16 MFMA route).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,6 +55,11 @@ constexpr int kPlanesMinMGroups32 = 5;
 // columns).
 hipError_t launch_cint8_planes(const CSegs& sg, const CInt8Launch& L, int m, int k, bool grouped,
                                hipStream_t s);
+
+// The projections of L on f16 MFMA (canonical_f16.hip).  All checks done by
+// the caller: 16-byte aligned codes, K % 64 == 0, not the RoPE mode; groups of
+// 32 or a multiple of 64 columns.
+hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k, hipStream_t s);
 
 // The call's scratch: buffer 0 of its stream's cache entry, whose call lock
 // `hold` keeps until the caller's last launch.

@@ -74,6 +74,17 @@ __device__ __forceinline__ void dma4(const void* base, uint32_t voff, const void
       : "v"(voff), "s"(base), "s"(m0)
       : "memory", "m0");
 }
+// Same with a per-lane 64-bit address.
+__device__ __forceinline__ void dma4_addr(const void* addr, const void* lds) {
+  const uint32_t m0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, off"
+      :
+      : "v"(addr), "s"(m0)
+      : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 }  // namespace qc

@@ -644,3 +644,119 @@ def test_cint8_row_plane_route_nonfinite_rows(qc, oracle, synth, dev):
         for got, want in ((np.isnan(Y[r]), np.isnan(y64)), (np.isposinf(Y[r]), np.isposinf(y64)),
                           (np.isneginf(Y[r]), np.isneginf(y64))):
             assert np.array_equal(got, want), (r, np.flatnonzero(got != want)[:5])
+
+
+# The f16 MFMA route: groups of 32 from 33 rows, other groups from 65, row
+# scales from 129 (small N) or past the row planes' K; tile edges along m and n,
+# K of one and of odd 64-column steps, and zero points: none, integers, and
+# some that are fractional or too large to take out of the codes.
+@pytest.mark.parametrize("m,rows,cols,gsize,zeros,swiglu", [
+    (33, 129, 64, 32, "none", False), (64, 300, 320, 32, "mixed", False),
+    (65, 31, 192, 64, "int", False), (129, 257, 64, 0, "int", False),
+    (200, 300, 448, 0, "mixed", True), (66, 1000, 1024, 128, "mixed", True),
+    (130, 128, 512, 256, "int", True), (513, 2049, 128, 64, "none", False),
+    (40, 96, 16448, 0, "mixed", False), (700, 5000, 64, 32, "int", True)])
+def test_cint8_f16_route(qc, oracle, dev, m, rows, cols, gsize, zeros, swiglu):
+    import torch
+    print(f"cint8 f16 m={m} rows={rows} cols={cols} gsize={gsize} zeros={zeros} "
+          f"swiglu={swiglu}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m + rows + cols)
+    groups = cols // gsize if gsize else 1
+    ws, what, keep = [], [], []
+    for _ in range(2 if swiglu else 1):
+        codes = torch.randint(-128, 128, (rows, cols), generator=g, device=dev, dtype=torch.int8)
+        scales = 1e-3 * (0.5 + torch.rand((rows, groups), generator=g, device=dev))
+        z = None
+        if zeros != "none":
+            z = torch.randint(-40, 40, (rows, groups), generator=g, device=dev).float()
+        if zeros == "mixed":
+            z[::3, -1] += 0.375
+            z[5::7, 0] = 5000.0
+            z[1::11, 0] = -1152.0
+        ws.append(qc.cint8_weights(codes, scales, z, rows, cols, groups))
+        keep.append((codes, scales, z))
+        q = codes.double().reshape(rows, groups, -1)
+        q = q if z is None else q - z.double()[:, :, None]
+        what.append((q * scales.double()[:, :, None]).reshape(rows, cols))
+    x = torch.randn((m, cols), generator=g, device=dev)
+    x[torch.rand((m, cols), generator=g, device=dev) < 0.01] *= 20.0
+    x[3] = 0.0
+    x[7] *= 1e-30
+    mode = 1 if swiglu else 0
+
+    def run(X, xt, yt=0, bad=()):
+        Y = torch.full((m, rows), float("nan"), device=dev) if yt == 0 else \
+            torch.zeros((m, rows), dtype=torch.int16, device=dev)
+        assert qc.cint8_project_raw(mode, ws, X, xt, m, [Y], [yt]) == 0
+        torch.cuda.synchronize()
+        return Y
+
+    def check(Y, X):
+        ys, bounds = [], []
+        for w in what:
+            ys.append(X.double() @ w.T.contiguous())
+            bounds.append(TOL * X.double().norm(dim=1, keepdim=True) * w.norm(dim=1)[None, :])
+        if not swiglu:
+            assert bool(((Y.double() - ys[0]).abs() <= bounds[0]).all())
+            return
+        # SiLU has slope at most 1.1; 1e-6 covers expf and the f32 products
+        silu = ys[0] / (1.0 + torch.exp(-ys[0]))
+        tol = 1.1 * bounds[0] * (ys[1].abs() + bounds[1]) + silu.abs() * bounds[1] + \
+            1e-6 * (silu * ys[1]).abs()
+        assert bool(((Y.double() - silu * ys[1]).abs() <= tol + 1e-30).all())
+
+    y = run(x, 0)
+    check(y, x)
+    assert torch.equal(y.view(torch.int32), run(x, 0).view(torch.int32))
+    # 16-bit outputs: the f32 values rounded once; 16-bit activations: the f32
+    # outputs of their decoded values
+    assert torch.equal(run(x, 0, 1), y.half().view(torch.int16))
+    assert torch.equal(run(x, 0, 2), y.bfloat16().view(torch.int16))
+    for t, dt in ((1, torch.float16), (2, torch.bfloat16)):
+        xh = x.to(dt)
+        yh = run(xh, t)
+        check(yh, xh.float())
+        assert torch.equal(yh.view(torch.int32), run(xh.float(), 0).view(torch.int32))
+    # rows holding NaN or +-inf: the class of the exact sum, other rows unchanged
+    xb = x.clone()
+    xb[0, 5] = float("inf")
+    xb[m - 1, cols - 1] = float("nan")
+    xb[20, 3] = float("-inf")
+    yb = run(xb, 0)
+    same = torch.ones(m, dtype=torch.bool, device=dev)
+    same[[0, 20, m - 1]] = False
+    assert torch.equal(yb[same].view(torch.int32), y[same].view(torch.int32))
+    assert bool(torch.isnan(yb[m - 1]).all())
+    if not swiglu:
+        for r in (0, 20):
+            want = (what[0] * xb[r].double()[None, :]).sum(dim=1)
+            assert torch.equal(torch.isnan(yb[r]), torch.isnan(want))
+            ok = ~torch.isnan(want)
+            assert bool((yb[r][ok].double() == want[ok]).all())
+
+
+def test_cint8_f16_route_epilogue(qc, oracle, dev):
+    """Bias and every activation at 300 rows, and three matrices over one x."""
+    import torch
+    m, rows, cols = 300, 200, 256
+    g = torch.Generator(device=dev).manual_seed(3)
+    mats = []
+    for r in (rows, 96, 33):
+        c = torch.randint(-127, 128, (r, cols), generator=g, device=dev, dtype=torch.int8)
+        s = 1e-2 * (0.5 + torch.rand((r, 1), generator=g, device=dev))
+        mats.append((c, s, qc.cint8_weights(c, s, None, r, cols, 1)))
+    x = torch.randn((m, cols), generator=g, device=dev)
+    ys = [torch.empty((m, c.shape[0]), device=dev) for c, _, _ in mats]
+    print("cint8 f16 epilogue", flush=True)
+    assert qc.cint8_project_raw(0, [w for _, _, w in mats], x, 0, m, ys, [0, 0, 0]) == 0
+    for (c, s, _), y in zip(mats, ys):
+        want = x.double() @ (c.double() * s.double()).T.contiguous()
+        bound = TOL * x.double().norm(dim=1, keepdim=True) * (c.double() * s.double()).norm(dim=1)
+        assert bool(((y.double() - want).abs() <= bound).all())
+    bias = torch.randn(rows, generator=g, device=dev)
+    for act in range(5):
+        y = torch.empty((m, rows), device=dev)
+        assert qc.cint8_project_raw(0, [mats[0][2]], x, 0, m, [y], [0], bias=bias,
+                                    activation=act) == 0
+        v = ys[0].double().cpu().numpy() + bias.double().cpu().numpy()[None, :]
+        assert np.allclose(y.cpu().numpy(), oracle.linear_activation_f64(v, act), rtol=1e-5, atol=1e-6)
