@@ -514,7 +514,15 @@ hipError_t launch_int8_gemm(const int8_t* W, const int8_t* X, const float* ws, c
       if (tiles(128, 128) >= cus * 3 / 4)
         return launch_ring<128, 128, 4, 2, 4>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
                                               asymmetric, status, s);
-      return launch_ring<64, 128, 4, 2, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
+      // Fewer workgroups than that: a K step is then mostly latency (barrier,
+      // LDS reads, loads), so the smallest tile that runs in one round, with
+      // two waves per SIMD for the larger of the two.  K = 4096, N = 4096,
+      // against 64 x 128 with four waves: M = 64 / 128 14.0 / 14.2 -> 9.7 / 10.0
+      // us (64 x 64), M = 301 16.1 -> 14.8, M = 512 17.4 -> 17.1 (128 x 64).
+      if (tiles(64, 64) <= cus)
+        return launch_ring<64, 64, 4, 2, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
+                                            asymmetric, status, s);
+      return launch_ring<128, 64, 4, 4, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
                                            asymmetric, status, s);
     }
     case kInt8Dma:

@@ -211,3 +211,25 @@ def test_validation_and_nonfinite_scales(qc, dev):
     assert qc.int8_gemm_raw(w, x, ws, as_, None, None, y, 1, 2, 64, dev_status=status) == 0
     torch.cuda.synchronize()
     assert int(status.item()) == 3
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 32), (63, 65, 96), (64, 4096, 4096), (129, 4033, 1056),
+                                   (301, 4096, 4128), (520, 3999, 160)])
+def test_small_ring_tiles(qc, dev, m, n, k):
+    """The automatic route's tiles for few workgroups (64 x 64 while they run
+    in one round, then 128 x 64), at their edges: exact accumulators, and the
+    epilogue's bits from them."""
+    import torch
+    print(f"int8 small tiles m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(m + n + k)
+    w = _t(rng.integers(-128, 128, (n, k), dtype=np.int8), dev)
+    x = _t(rng.integers(-128, 128, (m, k), dtype=np.int8), dev)
+    ws = _t(rng.uniform(1e-4, 1e-2, n).astype(np.float32), dev)
+    as_ = _t(rng.uniform(1e-3, 1e-1, m).astype(np.float32), dev)
+    zp = _t(rng.integers(-128, 128, m).astype(np.int32), dev)
+    rs = w.sum(1, dtype=torch.int32)
+    acc = x.double() @ w.double().T.contiguous()
+    assert torch.equal(qc.int8_gemm_i32(w, x).double(), acc)
+    y = qc.int8_gemm(w, x, ws, as_, rs, zp, True)
+    want = ((acc - zp.double()[:, None] * rs.double()[None, :]).float() * ws[None, :]) * as_[:, None]
+    assert torch.equal(y.view(torch.int32), want.view(torch.int32))
