@@ -18,6 +18,7 @@
 // staged per workgroup into LDS (padded by 16 B every 64 floats so the per-
 // lane 256-B slices of consecutive lanes fall into different banks) and every
 // decoded weight is reused for up to 8 activation rows.
+#include <atomic>
 #include "qc_device.h"
 #include "qc_internal.h"
 
@@ -315,13 +316,18 @@ hipError_t launch_qgemm(int fmt, const void* W, const float* x, float* y, long l
 }
 
 // Compute units of the current device (256 on a full MI355X; fewer under a
-// compute partition).  The tile and split planners size their grids by it.
+// compute partition).  The tile and split planners size their grids by it, on
+// every call: the attribute is looked up once per device.
 int device_cu_count() {
+  constexpr int kDevices = 64;
+  static std::atomic<int> known[kDevices];
   int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+  if (dev < kDevices && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       cus <= 0)
-    cus = 256;
+    return 256;
+  if (dev < kDevices) known[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
 

@@ -87,15 +87,30 @@ class QcError(RuntimeError):
         self.status = status
 
 
+# A pointer argument is declared c_void_p, so a plain int is passed as it is; a
+# one-projection call spends several us here, as long as its kernel, when every
+# pointer is wrapped and the current stream looked up as a Stream object.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = None   # current stream handle of the current device
 
 
 def _stream(stream):
     if stream is not None:
-        return ctypes.c_void_p(stream)
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return stream
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()   # initialises the device
+        c = torch._C
+        if hasattr(c, "_cuda_getCurrentRawStream") and hasattr(c, "_cuda_getDevice"):
+            raw, device = c._cuda_getCurrentRawStream, c._cuda_getDevice
+            _raw_stream = lambda: raw(device())
+        else:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream
+    return _raw_stream()
 
 
 def _check(status, what):
