@@ -359,7 +359,7 @@ int qc_hip_set_int8_gemm_route(int route);
 int qc_hip_set_qgemm_plan(int waves, int stages);
 
 /* Route of qc_hip_qgemm for M >= 2 (K % 64 == 0): 0 (the default) runs the
- * 2-D tiled GEMM for M >= 33 and one pass of at most 32 rows below; -1 always
+ * 2-D tiled GEMM for M >= 33 (q4_0: 17) and one pass below; -1 always
  * uses the passes; 1 / 2 always use the 2-D GEMM with one / two K ranges.
  * Results stay within the contract tolerance on every route.  Tuning and
  * test knob with no reference counterpart. */

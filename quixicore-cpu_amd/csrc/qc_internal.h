@@ -42,7 +42,7 @@ struct GemvTuning {
   int rows_per_wave = 0;  // GEMV rows per wavefront (1, 2, 4, 7, 8, 14; 0 = from the shape)
   int qgemm_waves = 0;    // small-batch GEMM waves per workgroup (4, 8; 0 = from the shape)
   int qgemm_stages = 0;   // small-batch GEMM K stages per workgroup (1..16; 0 = from the shape)
-  int qgemm_panel = 0;    // 2-D GEMM route: 0 = for m >= 33, -1 = never, 1 / 2 = always (K ranges)
+  int qgemm_panel = 0;    // 2-D GEMM route: 0 = for m >= 33 (q4_0: 17), -1 = never, 1 / 2 = always (K ranges)
   int qgemm_rows = 0;     // exact-digit rows route for 2 <= m <= 8: 0 = by shape, -1 = never, 1 = always
   int qgemm_fold = 0;     // digit-layout GEMM builds its own digits: 0 = where it can, -1 = never
   int cint8_dot = 0;      // canonical int8, M = 1: digit-dot kernel 0 = where it applies, -1 = never
@@ -95,7 +95,7 @@ hipError_t launch_qgemv_w8a8(int fmt, const void* W, const float* x, float* y, l
                              long long k, int rows_per_wave, int* status, hipStream_t s);
 
 // GEMM on MFMA (m >= 2, K % 64 == 0, W 4-byte aligned): int8 digit planes
-// for up to 8 rows per pass, f16 / bf16 hi/lo above; from 33 rows one 2-D
+// for up to 8 rows per pass, f16 / bf16 hi/lo above; from 33 rows (q4_0: 17) one 2-D
 // tiled GEMM (launch_qgemm_wide) instead of passes of 32 rows.  waves / stages:
 // small-batch plan override (0 = from the shape); panel: 0 = from m, -1 =
 // never, 1 / 2 = always (one / two K ranges).  fold: 0 = the digit-layout

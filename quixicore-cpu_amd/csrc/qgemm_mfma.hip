@@ -1,7 +1,7 @@
 // Small-batch q8_0 / q4_0 GEMM (2 <= M, in tiles of 16 activation rows) on
 // gfx950 MFMA: int8 digit planes for up to 8 rows per pass, f16 (q8_0) or
-// bf16 (q4_0) operands above.  From 33 rows a call takes the 2-D tiled GEMMs
-// (qgemm_wide.hip, qgemm_mx.hip) instead of passes of 32.
+// bf16 (q4_0) operands above.  From 33 rows (q4_0: 17) a call takes the 2-D
+// tiled GEMMs (qgemm_wide.hip, qgemm_mx.hip) instead of passes of 32.
 //
 // Semantics as the reference's qgemm (kernels/quantization/qgemm_ref.cpp:
 // 156-162, one qgemv per activation row: y[m][n] = sum_b d[n][b] *
@@ -1182,10 +1182,15 @@ hipError_t qgemm_mfma_with(int fmt, const void* W, const float* x, float* y, int
                            hipStream_t s, int waves, int stages, int panel, Scratch& scratch) {
   const auto* w = static_cast<const uint8_t*>(W);
   // panel: 0 = from m, -1 = never, 1 / 2 = always (for m >= 2) with one / two
-  // K ranges.  From 33 rows a pass of 32 would stream the weights twice.  A
-  // forced small-batch plan keeps the passes below 64 rows.
+  // K ranges.  From 33 rows a pass of 32 would stream the weights twice.  For
+  // q4_0 its 32-row tile is the faster from 17 rows (M = 32, pass / tile:
+  // N = 4096, K = 1024 11.0 / 10.9 us; N = 14336, K = 4096 28.0 / 24.9;
+  // N = 28672, K = 14336 172 / 111; M = 17, N = 14336 26.7 / 24.4); at 16 rows
+  // the pass is (20.5 / 23.6), and for q8_0 the two are within 6% either way.
+  // A forced small-batch plan keeps the passes below 64 rows.
   const bool forced = waves != 0 || stages != 0;
-  if (scratch.w != nullptr && (panel > 0 || (panel == 0 && m > (forced ? 63 : 32))))
+  const int wide_from = forced ? 64 : fmt == kQ4_0 ? 17 : 33;
+  if (scratch.w != nullptr && (panel > 0 || (panel == 0 && m >= wide_from)))
     return launch_qgemm_wide(fmt, W, x, y, m, n, k, panel, s, scratch.w);
   // The f16 / bf16 layouts (passes of more than 8 rows) scale each row by its
   // power of two; their prep kernel stores the exponents here.

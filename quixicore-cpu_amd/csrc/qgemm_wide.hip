@@ -21,7 +21,11 @@
 // reads, the next block's decode and the ring's loads, in fixed order.
 // q8_0, N = 14336, K = 4096, M = 2048: 602 -> 467 us (515 TFLOP/s; a plain f16
 // GEMM of this chip reaches 1430, and this is two products); M = 77, N = 5461,
-// K = 2752: 51.7 -> 24.5 us (three passes of 32 rows before).
+// K = 2752: 51.7 -> 24.5 us (three passes of 32 rows before).  For 17-32 rows
+// (q4_0) a 32 x 128 tile of four waves: what bounds it there is the activation
+// fragments, which every workgroup reads whole (57 MB from L2 at N = 14336,
+// K = 4096, beside 33 MB of weights): 28.0 -> 24.4 us; N = 28672, K = 14336
+// 172 -> 111 us.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -335,7 +339,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
     // Barrier B_s stands before the last m-tile of step s.  Step s issues,
     // before B_s, x step s + XR - 1 and (s odd) weight pair (s - 1) / 2 + WR;
     // at B_s only the loads of the last XR - 2 steps may be outstanding, so x
-    // step s + 1 and the weights of block s + 2 are in.
+    // step s + 1 and the weights of block s + 2 are in.  With one m-tile B_s
+    // opens step s, whose loads follow it (into x slot s - 1, last read before
+    // B_{s-1}): the loads of the last XR - 3 steps may then be outstanding.
     auto load_w = [&](int slot) {
 #pragma unroll
       for (int i = 0; i < C::WL; ++i) issue_w1(slot, i);
@@ -399,8 +405,12 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
         const Weights& cur = tn < NE ? we[kOdd ? 1 : 0][tn < NE ? tn : 0] : wl;
         const int ab = ((kOdd ? TM : 0) + tm) & 1;     // operand buffer of this m-tile
         const int pi = i == 0 ? T - 1 : i - 1, pm = pi / TN, pn = pi % TN;
+        const int cb = ((kOdd ? T : 0) + i) & 1;       // result buffer
         if (i == B) {
-          wait_vmcnt<(XR - 2) * C::XL + (kOdd ? XR - 1 : XR - 3) / 2 * C::WL>();
+          if constexpr (B > 0)
+            wait_vmcnt<(XR - 2) * C::XL + (kOdd ? XR - 1 : XR - 3) / 2 * C::WL>();
+          else                                     // this step's loads go out after B_s
+            wait_vmcnt<(XR - 3) * C::XL + (XR - 3) / 2 * C::WL>();
           wait_lgkmcnt0();
           ring_barrier();
         }
@@ -410,14 +420,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
           // the last n-tile takes operands 2, 3 first: they are then free
           // for the next m-tile's
           const int o = TN > 1 && tn == TN - 1 ? q ^ 2 : q;
-          c[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o < 2 ? ae[ab][o & 1] : al[o & 1],
-                                                            cur.w[o >> 1],
-                                                            q == 0 ? z : c[i & 1], 0, 0, 0);
+          c[cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(o < 2 ? ae[ab][o & 1] : al[o & 1],
+                                                         cur.w[o >> 1], q == 0 ? z : c[cb], 0, 0, 0);
           // the previous tile's last MFMA is still running in slot 0
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int e = q == 0 ? 0 : 16 * (q - 1) / 3; e < 16 * q / 3; ++e)
-            acc[pm][pn][e] = fmaf(c[(i & 1) ^ 1][e], dprev, acc[pm][pn][e]);
+            acc[pm][pn][e] = fmaf(c[cb ^ 1][e], dprev, acc[pm][pn][e]);
           const int ms = 4 * tn + q, slot = 4 * i + q;
           // the next m-tile's operands: 0 and 1 early, 2 and 3 after their last use
           const uint8_t* nx = tm + 1 < TM ? xw + xs * C::XS + (tm + 1) * kStepBytes
@@ -426,9 +435,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
             ae[ab ^ 1][ms / TN] = *reinterpret_cast<const f16x8*>(nx + ms / TN * 1024);
           if (tn == TN - 1 && o >= 2)
             al[o & 1] = *reinterpret_cast<const f16x8*>(nx + o * 1024);
-          if (i < B) {
+          constexpr int kIssue = 4 * (B > 0 ? B : T);    // slots that issue loads
+          if (slot < kIssue) {
 #pragma unroll
-            for (int l = slot * NL / (4 * B); l < (slot + 1) * NL / (4 * B); ++l) issue(l);
+            for (int l = slot * NL / kIssue; l < (slot + 1) * NL / kIssue; ++l) issue(l);
           }
           // weights: read n-tile by n-tile (well before B_s, which waits for
           // LDS reads), decoded a dword at a time
@@ -461,7 +471,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
     }
 #pragma unroll
     for (int e = 0; e < 16; ++e)
-      acc[TM - 1][TN - 1][e] = fmaf(c[(TM * TN - 1) & 1][e], dprev, acc[TM - 1][TN - 1][e]);
+      acc[TM - 1][TN - 1][e] = fmaf(c[1][e], dprev, acc[TM - 1][TN - 1][e]);
   }
   wait_vmcnt<0>();   // no global->LDS load may outlive the workgroup's LDS
 
@@ -475,12 +485,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
 // Times per block pair, measured on MI355X with q8_0 at K = 4096 (q4_0 within
 // 10%): 256 x 256 tiles 182 us for 112 workgroups, 467 for 448; 128 x 256
 // 129 us for 224, 538 for 896; 128 x 128 145 us for 448; 64 x 128 30 us for
-// 128 half-K workgroups.
-constexpr int kTiles = 4;
-constexpr Tile kTile[kTiles] = {{256, 256, 1, 2.84, 4.10},
+// 128 half-K workgroups.  Up to 32 rows take the last tile alone (q4_0,
+// K = 14336: 98 us for 16 workgroups, 111 for 224): a workgroup more than there
+// are CUs costs a round (two share a CU's operand feed), and its ring is nine
+// steps deep, because a step is only one MFMA tile (N = 14336, K = 4096, two K
+// ranges: 25.7 us with seven steps, 24.4 with nine, 25.5 with fifteen).
+constexpr int kTiles = 4;   // for more than 32 rows
+constexpr Tile kTile[kTiles + 1] = {{256, 256, 1, 2.84, 4.10},
                                 {128, 256, 1, 1.70, 2.30},
-                                {128, 128, 2, 1.10, 2.44},
-                                {64, 128, 1, 0.48, 0.68}};
+                                    {128, 128, 2, 1.10, 2.44},
+                                    {64, 128, 1, 0.48, 0.68},
+                                    {32, 128, 1, 0.42, 0.48}};
 
 template <int FMT, int TM, int TN, int WGM, int WGN, int XR>
 hipError_t launch_tile(const uint8_t* W, const uint8_t* xf, float* y, float* partial,
@@ -497,9 +512,12 @@ template <int FMT>
 hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, int k, int ranges,
                     hipStream_t s, StreamWorkspace* ws) {
   const int nb = k / 32;
-  const TilePlan p = plan_tiles(kTile, kTiles, m, n, k / 64, device_cu_count(), ranges, 8);
+  TilePlan p = m <= 32 ? plan_tiles(&kTile[kTiles], 1, m, n, k / 64, device_cu_count(), ranges, 8)
+                       : plan_tiles(kTile, kTiles, m, n, k / 64, device_cu_count(), ranges, 8);
+  if (m <= 32) p.tile = kTiles;
   const long long outs = static_cast<long long>(m) * n;
-  const size_t xf_bytes = static_cast<size_t>((m + 255) / 256 * 8) * nb * kStepBytes;
+  const int mtiles = m <= 32 ? 1 : (m + 255) / 256 * 8;
+  const size_t xf_bytes = static_cast<size_t>(mtiles) * nb * kStepBytes;
   const size_t part_bytes = p.ks > 2 ? static_cast<size_t>(p.ks) * outs * sizeof(float) : 0;
   void* buf = nullptr;
   hipError_t e = stream_buffer(ws, s, xf_bytes + part_bytes, 0, &buf);
@@ -527,7 +545,8 @@ hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, in
     case 0: e = launch_tile<FMT, 4, 2, 2, 4, 3>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
     case 1: e = launch_tile<FMT, 2, 2, 2, 4, 3>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
     case 2: e = launch_tile<FMT, 2, 2, 2, 2, 3>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
-    default: e = launch_tile<FMT, 2, 1, 1, 4, 5>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
+    case 3: e = launch_tile<FMT, 2, 1, 1, 4, 5>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
+    default: e = launch_tile<FMT, 1, 1, 1, 4, 9>(W, xf, y, partial, rexp, x, m, n, k, p, s); break;
   }
   if (e != hipSuccess || p.ks <= 2) return e;
   wide_reduce<<<static_cast<unsigned>(std::min<long long>(4096, (outs + 255) / 256)), 256, 0, s>>>(

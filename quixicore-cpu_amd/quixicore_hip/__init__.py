@@ -343,7 +343,7 @@ def set_qgemm_plan(waves=0, stages=0):
 
 
 def set_qgemm_panel(mode=0):
-    """qgemm route for M >= 2: 0 = 2-D GEMM for M >= 33, -1 = never,
+    """qgemm route for M >= 2: 0 = 2-D GEMM for M >= 33 (q4_0: 17), -1 = never,
     1 / 2 = always with one / two K ranges."""
     _check(lib.qc_hip_set_qgemm_panel(mode), "set_qgemm_panel")
 

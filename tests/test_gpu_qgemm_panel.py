@@ -96,12 +96,14 @@ def test_panel_prefill_sizes(qc, oracle, dev, fmt, m, n, k):
     _check(oracle, fmt, P.cpu().numpy(), x, y, n, k, (0, 1, m // 2, m - 1))
 
 
-# Automatic route: 33 rows is the first 2-D call, and shapes around the edges
-# of its tiles (64 / 128 / 256 rows by 128 / 256 columns), with K of one block
+# Automatic route: 33 rows (q4_0: 17) are the first 2-D call, and shapes around the edges
+# of its tiles (32 / 64 / 128 / 256 rows by 128 / 256 columns), with K of one block
 # pair, odd pairs, and K splits; from 384 rows and 2048 columns q4_0 takes the
 # re-encoded 6-bit form.
 @pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("m,n,k", [(33, 129, 64), (64, 2048, 4096), (65, 127, 320),
+@pytest.mark.parametrize("m,n,k", [(17, 129, 64), (18, 127, 320), (31, 1361, 1088),
+                                   (32, 4096, 4096), (32, 14337, 512),
+                                   (33, 129, 64), (64, 2048, 4096), (65, 127, 320),
                                    (77, 1361, 1088), (257, 300, 448), (383, 2049, 192),
                                    (384, 2048, 64), (385, 2079, 576), (641, 2305, 128),
                                    (1025, 4097, 192), (2049, 2080, 64)])
