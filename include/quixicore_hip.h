@@ -97,9 +97,8 @@ int qc_hip_qgemm(int format, const void* packed, const float* x, float* y, long 
  * first launch to its last, so calls from several host threads on ONE stream
  * are safe (their launch sequences queue one after the other); calls on
  * different streams of one GPU can overlap on the device and race: serialize
- * those.  M >= 2 runs passes of at
- * most 32 rows (never the 2-D route, whose scratch grows with m) with
- * the fewest K splits.  Limits: m <= QC_QGEMM_NOALLOC_MAX_M and
+ * those.  M > 32 runs passes of at most 32 rows (not the 2-D route's larger
+ * tiles, whose scratch grows with m), and passes take the fewest K splits.  Limits: m <= QC_QGEMM_NOALLOC_MAX_M and
  * k <= QC_QGEMM_NOALLOC_MAX_K, else 1 (QC_INVALID_SHAPE) with a message in
  * qc_hip_last_error().  Within k <= 8192 every such call fits; above it, a
  * call whose K-split partial sums (ceil(k/4096) * min(m, 32) * n * 4 bytes)

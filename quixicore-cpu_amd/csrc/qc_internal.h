@@ -38,6 +38,30 @@ struct StreamWorkspace {
 hipError_t stream_workspace(hipStream_t s, StreamWorkspace** out);
 hipError_t stream_buffer(StreamWorkspace* w, hipStream_t s, size_t bytes, int tag, void** out);
 
+// Where a call's scratch comes from: a per-stream cache entry (whose `call`
+// lock the caller holds), or a fixed region given by the caller -- region 1
+// at [0, fixed_split), region 0 at [fixed_split, fixed_bytes).  A fixed
+// region never grows: a request beyond it fails with hipErrorOutOfMemory
+// before anything is launched (the first pass of a call needs the most).
+struct Scratch {
+  StreamWorkspace* w = nullptr;
+  uint8_t* fixed = nullptr;
+  size_t fixed_split = 0, fixed_bytes = 0;
+  int max_ks = 0;   // > 0: K split limit for the small-batch plan (see plan_for)
+  int fold = 0;     // digit layouts: 0 = build the digits in the GEMM where it can, -1 = never
+
+  hipError_t get(hipStream_t s, size_t bytes, void** out, int tag = 0) {
+    if (w == nullptr) {
+      const size_t lo = tag == 1 ? 0 : fixed_split;
+      const size_t hi = tag == 1 ? fixed_split : fixed_bytes;
+      if (bytes > hi - lo) return hipErrorOutOfMemory;
+      *out = fixed + lo;
+      return hipSuccess;
+    }
+    return stream_buffer(w, s, bytes, tag, out);
+  }
+};
+
 struct GemvTuning {
   int rows_per_wave = 0;  // GEMV rows per wavefront (1, 2, 4, 7, 8, 14; 0 = from the shape)
   int qgemm_waves = 0;    // small-batch GEMM waves per workgroup (4, 8; 0 = from the shape)
@@ -106,9 +130,10 @@ hipError_t launch_qgemm_mfma(int fmt, const void* W, const float* x, float* y, i
 
 // The 2-D tiled route of launch_qgemm_mfma (m >= 2, K % 64 == 0, W 4-byte
 // aligned): f16 MFMA over hi / lo activations.  ranges: K ranges, 0 = from
-// the shape.  The caller holds ws->call.
+// the shape.  The caller holds the scratch's call lock; more than 32 rows take
+// a cache entry's scratch.
 hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, int m, int n,
-                             int k, int ranges, hipStream_t s, StreamWorkspace* ws);
+                             int k, int ranges, hipStream_t s, Scratch& scratch);
 
 // The q4_0 form of it that re-encodes weights and activations for the
 // block-scaled 6-bit MFMA, and the sizes it is taken for.

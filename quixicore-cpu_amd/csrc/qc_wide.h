@@ -147,9 +147,10 @@ struct TilePlan {
 };
 // ranges: the K ranges wanted, 0 = any up to max_ks.  Two ranges add into a
 // cleared y (2048 x 4096 outputs: about 45 us more than stores); more are
-// summed from partial outputs by a second launch (4 bytes / ps).
+// summed from partial outputs, of at most max_partial bytes, by a second launch
+// (4 bytes / ps).
 inline TilePlan plan_tiles(const Tile* tiles, int count, int m, int n, int units, int cus,
-                           int ranges, int max_ks) {
+                           int ranges, int max_ks, double max_partial = 256e6) {
   TilePlan best;
   const double bytes = 4.0 * m * n;
   for (int i = 0; i < count; ++i) {
@@ -159,7 +160,7 @@ inline TilePlan plan_tiles(const Tile* tiles, int count, int m, int n, int units
       if (ranges > 0 ? want != std::min(ranges, units) : want > max_ks) continue;
       const int per = (units + want - 1) / want;
       const int ks = (units + per - 1) / per;
-      if (ks != want || (ks > 2 && ks * bytes > 256e6)) continue;
+      if (ks != want || (ks > 2 && ks * bytes > max_partial)) continue;
       const double rounds = wgs * ks / (static_cast<double>(cus) * c.slots);
       const double us = std::max(std::ceil(rounds) * (per * c.alone_us + 2.0),
                                  rounds * per * c.full_us + 2.0) +

@@ -987,30 +987,6 @@ __global__ __launch_bounds__(64 * NW * KG) void qgemm_mfma(
 // entry points take buffers 0 and 1 of the stream's cache entry
 // (stream_workspace, qc_internal.h).
 //
-// Where a call's scratch comes from: a per-stream cache entry (whose `call`
-// lock the caller holds), or a fixed region given by the caller -- region 1
-// at [0, fixed_split), region 0 at [fixed_split, fixed_bytes).  A fixed
-// region never grows: a request beyond it fails with hipErrorOutOfMemory
-// before anything is launched (the first pass of a call needs the most).
-struct Scratch {
-  StreamWorkspace* w = nullptr;
-  uint8_t* fixed = nullptr;
-  size_t fixed_split = 0, fixed_bytes = 0;
-  int max_ks = 0;   // > 0: K split limit for the small-batch plan (see plan_for)
-  int fold = 0;     // digit layouts: 0 = build the digits in the GEMM where it can, -1 = never
-
-  hipError_t get(hipStream_t s, size_t bytes, void** out, int tag = 0) {
-    if (w == nullptr) {
-      const size_t lo = tag == 1 ? 0 : fixed_split;
-      const size_t hi = tag == 1 ? fixed_split : fixed_bytes;
-      if (bytes > hi - lo) return hipErrorOutOfMemory;
-      *out = fixed + lo;
-      return hipSuccess;
-    }
-    return stream_buffer(w, s, bytes, tag, out);
-  }
-};
-
 struct MfmaArgs {
   const uint8_t* W;
   const uint8_t* xf;
@@ -1190,8 +1166,10 @@ hipError_t qgemm_mfma_with(int fmt, const void* W, const float* x, float* y, int
   // A forced small-batch plan keeps the passes below 64 rows.
   const bool forced = waves != 0 || stages != 0;
   const int wide_from = forced ? 64 : fmt == kQ4_0 ? 17 : 33;
-  if (scratch.w != nullptr && (panel > 0 || (panel == 0 && m >= wide_from)))
-    return launch_qgemm_wide(fmt, W, x, y, m, n, k, panel, s, scratch.w);
+  // The fixed region holds the fragments of 32 rows of up to 8192 columns and
+  // two K ranges of any n; above, a pass that does not fit is refused.
+  if ((scratch.w != nullptr || (m <= 32 && k <= 8192)) && (panel > 0 || (panel == 0 && m >= wide_from)))
+    return launch_qgemm_wide(fmt, W, x, y, m, n, k, panel, s, scratch);
   // The f16 / bf16 layouts (passes of more than 8 rows) scale each row by its
   // power of two; their prep kernel stores the exponents here.
   int* rexp = nullptr;
@@ -1289,8 +1267,7 @@ hipError_t launch_qgemm_mfma_noalloc(int fmt, const void* W, const float* x, flo
   scratch.max_ks = 2;
   if (scratch.fixed_split >= scratch.fixed_bytes) return hipErrorOutOfMemory;
   std::lock_guard<std::mutex> hold(d->call);   // until the call's last launch
-  // passes of at most 32 rows: the 2-D route's fragments grow with m
-  return qgemm_mfma_with(fmt, W, x, y, m, n, k, s, 0, 0, -1, scratch);
+  return qgemm_mfma_with(fmt, W, x, y, m, n, k, s, 0, 0, 0, scratch);
 }
 
 }  // namespace qc

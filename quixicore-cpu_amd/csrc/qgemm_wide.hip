@@ -510,22 +510,26 @@ hipError_t launch_tile(const uint8_t* W, const uint8_t* xf, float* y, float* par
 
 template <int FMT>
 hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, int k, int ranges,
-                    hipStream_t s, StreamWorkspace* ws) {
+                    hipStream_t s, Scratch& scratch) {
   const int nb = k / 32;
-  TilePlan p = m <= 32 ? plan_tiles(&kTile[kTiles], 1, m, n, k / 64, device_cu_count(), ranges, 8)
-                       : plan_tiles(kTile, kTiles, m, n, k / 64, device_cu_count(), ranges, 8);
-  if (m <= 32) p.tile = kTiles;
-  const long long outs = static_cast<long long>(m) * n;
   const int mtiles = m <= 32 ? 1 : (m + 255) / 256 * 8;
   const size_t xf_bytes = static_cast<size_t>(mtiles) * nb * kStepBytes;
+  const double left = scratch.w != nullptr ? 256e6
+                                           : static_cast<double>(scratch.fixed_bytes) -
+                                                 static_cast<double>(scratch.fixed_split + xf_bytes);
+  const int cus = device_cu_count();
+  TilePlan p = m <= 32 ? plan_tiles(&kTile[kTiles], 1, m, n, k / 64, cus, ranges, 8, left)
+                       : plan_tiles(kTile, kTiles, m, n, k / 64, cus, ranges, 8, left);
+  if (m <= 32) p.tile = kTiles;
+  const long long outs = static_cast<long long>(m) * n;
   const size_t part_bytes = p.ks > 2 ? static_cast<size_t>(p.ks) * outs * sizeof(float) : 0;
   void* buf = nullptr;
-  hipError_t e = stream_buffer(ws, s, xf_bytes + part_bytes, 0, &buf);
+  hipError_t e = scratch.get(s, xf_bytes + part_bytes, &buf);
   if (e != hipSuccess) return e;
   uint8_t* xf = static_cast<uint8_t*>(buf);
   float* partial = reinterpret_cast<float*>(xf + xf_bytes);
   // read in whole tiles: padded to the largest
-  e = stream_buffer(ws, s, sizeof(int) * static_cast<size_t>((m + 255) / 256 * 256), 1, &buf);
+  e = scratch.get(s, sizeof(int) * 32 * static_cast<size_t>(mtiles), &buf, 1);
   if (e != hipSuccess) return e;
   int* rexp = static_cast<int*>(buf);
 
@@ -557,9 +561,9 @@ hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, in
 }  // namespace
 
 hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, int m, int n, int k,
-                             int ranges, hipStream_t s, StreamWorkspace* ws) {
+                             int ranges, hipStream_t s, Scratch& scratch) {
   const auto* w = static_cast<const uint8_t*>(W);
-  if (fmt == kQ4_0 && ranges == 0 && mx_pays(m, n)) return launch_qgemm_mx(W, x, y, m, n, k, s, ws);
+  if (fmt == kQ4_0 && ranges == 0 && mx_pays(m, n)) return launch_qgemm_mx(W, x, y, m, n, k, s, scratch.w);
   // Rows in chunks whose fragments (4 bytes an element) take at most 256 MB.
   const long long fit = (256LL << 20) / (4LL * k) / 256 * 256;
   const int chunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, INT_MAX / 2)));
@@ -567,8 +571,8 @@ hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, i
     const int mc = std::min(chunk, m - m0);
     const float* xm = x + static_cast<long long>(m0) * k;
     float* ym = y + static_cast<long long>(m0) * n;
-    const hipError_t e = fmt == kQ8_0 ? run_wide<kQ8_0>(w, xm, ym, mc, n, k, ranges, s, ws)
-                                      : run_wide<kQ4_0>(w, xm, ym, mc, n, k, ranges, s, ws);
+    const hipError_t e = fmt == kQ8_0 ? run_wide<kQ8_0>(w, xm, ym, mc, n, k, ranges, s, scratch)
+                                      : run_wide<kQ4_0>(w, xm, ym, mc, n, k, ranges, s, scratch);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
