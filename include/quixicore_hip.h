@@ -379,8 +379,9 @@ int qc_hip_set_qgemm_rows(int mode);
  * the int8 MFMA GEMM, an exact combination per row or per group; K % 32 == 0,
  * K <= 16384, codes 16-byte aligned, not the RoPE mode); from some tens of
  * rows, where it measured faster, on f16 MFMA over the codes (K % 64 == 0:
- * groups of 32 from 33 rows, of a multiple of 64 from 65, row scales from 129
- * rows at small N); everything else on
+ * groups of 32 from 33 rows with zero points and 65 without, of 64 from 65, of a
+ * multiple of 128 from 65 with and at large M x N without, row scales from 129 rows
+ * at small N); everything else on
  * the kernels with exact int8 digit dots per 32-element block (the GEMV's
  * encoding of x) where they apply (K % 64 == 0, codes 16-byte aligned, row
  * scales or groups of >= 32 columns); 1 = never the row-plane route; -1 =

@@ -857,20 +857,26 @@ hipError_t launch_cint8(const CInt8Launch& L, hipStream_t s) {
   for (int i = 0; i < L.nw; ++i)
     fast = fast && reinterpret_cast<uintptr_t>(L.w[i].codes) % 16 == 0;
   // From some tens of rows: f16 MFMA where it measured faster than the row
-  // planes (K = 4096, us, planes / f16 with 16-bit and f32 activations).  Groups
-  // of 32, from 33 rows: N = 4096 M = 33 101 / 50, M = 128 150 / 53; N = 14336
-  // M = 512 586 / 151.  Other groups, from 65 rows: groups of 128 N = 4096 M =
-  // 64 43 / 46 and 52, M = 128 67 / 46 and 54; N = 14336 M = 128 75 / 59 and
-  // 64, M = 512 257 / 120 and 155.  Row scales from 129 rows while the planes'
+  // planes (K = 4096, us, planes / f16 with 16-bit and f32 activations); the
+  // planes' fold is much shorter without zero points.  Groups of 32 with zero
+  // points from 33 rows: N = 4096 M = 33 101 / 50 and 58; without from 65: N =
+  // 14336 M = 64 57 / 56 and 62, M = 65 80 / 56 and 63.  Groups of 64 from 65
+  // rows: N = 14336 M = 65 71 / 50 and 59.  Larger groups with zero points from
+  // 65: N = 4096 M = 64 43 / 46 and 52, M = 128 67 / 46 and 54; N = 14336 M = 128
+  // 75 / 59 and 64, M = 512 257 / 120 and 155; without where the planes' 64 x 128
+  // tiles take more than two rounds of the CUs: N = 14336 M = 128 (224 tiles) 55
+  // / 51 and 59, M = 256 (448) 101 / 89 and 109, SwiGLU M = 128 (448) 98 / 94
+  // and 107, M = 129 (672) 140 / - and 135, M = 512 (896) 199 / 120 and 155.  Row scales from 129 rows while the planes'
   // 64 x 256 output tiles fill at most half of the CUs: N = 4096 M = 256 60 /
   // 37 and 47, M = 512 63 / 41 and 54; N = 14336 M = 256 67 / 70 and 95.  (Every
   // rule is the same for f32 and 16-bit activations, whose results have the
   // same bits.)  Lengths the planes do not take go here as well.
   const long long plane_tiles = (m + 63LL) / 64 * ((L.w[0].rows * (L.mode == 1 ? 2 : 1) + 255) / 256);
   const bool planes_fit = k <= kPlanesMaxK && (!grp || k % 128 == 0);
-  const bool f16_pays = !grp              ? m > 128 && 2 * plane_tiles <= device_cu_count()
-                        : sg.gsize == 32 ? m > 32
-                                         : m > 64;
+  const bool f16_pays = !grp ? m > 128 && 2 * plane_tiles <= device_cu_count()
+                        : sg.gsize == 32 ? m > (aff ? 32 : 64)
+                        : sg.gsize == 64 ? m > 64
+                                         : m > 64 && (aff || plane_tiles > device_cu_count());
   if (fast && L.dot == 0 && L.mode != 2 && k % 64 == 0 &&
       (!grp || sg.gsize == 32 || sg.gsize % 64 == 0) && (f16_pays || (!planes_fit && m > 32)))
     return launch_cint8_f16(sg, L, m, k, s);

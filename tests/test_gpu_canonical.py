@@ -646,12 +646,13 @@ def test_cint8_row_plane_route_nonfinite_rows(qc, oracle, synth, dev):
             assert np.array_equal(got, want), (r, np.flatnonzero(got != want)[:5])
 
 
-# The f16 MFMA route: groups of 32 from 33 rows, other groups from 65, row
-# scales from 129 (small N) or past the row planes' K; tile edges along m and n,
+# The f16 MFMA route: groups of 32 from 33 rows (65 without zero points), other
+# groups from 65 (those over 64 without zero points past two rounds of tiles), row scales from 129 (small N) or past the row planes' K; tile edges along m and n,
 # K of one and of odd 64-column steps, and zero points: none, integers, and
 # some that are fractional or too large to take out of the codes.
 @pytest.mark.parametrize("m,rows,cols,gsize,zeros,swiglu", [
-    (33, 129, 64, 32, "none", False), (64, 300, 320, 32, "mixed", False),
+    (33, 129, 64, 32, "int", False), (64, 300, 320, 32, "mixed", False),
+    (65, 129, 64, 32, "none", False), (513, 8300, 128, 128, "none", False),
     (65, 31, 192, 64, "int", False), (129, 257, 64, 0, "int", False),
     (200, 300, 448, 0, "mixed", True), (66, 1000, 1024, 128, "mixed", True),
     (130, 128, 512, 256, "int", True), (513, 2049, 128, 64, "none", False),
