@@ -6,22 +6,38 @@
 // y[m][n] = sum_b d[n][b] * sum_{k in b} q[n][k] * x[m][k].
 //
 // Numerics.  q4_0 codes (-8..7) are exact in E2M3.  Each activation of a
-// 32-element block becomes four E2M3 digits at scales 2^-5 apart under the
-// block's own exponent: x - sum of digits is within 2^-20 of the block's
-// largest element, and the digits' scales are the instruction's own block
-// scales.  v_mfma_scale_f32_32x32x64_f8f6f4 with E2M3 operands multiplies two
-// digits of 32 elements at once (the digits are its two K halves, against the
-// same codes twice), so a block of a 32 x 32 tile is two MFMAs, half of the f16
-// form's four, folded into the f32 accumulators by one FMA per output with
-// the block's scale.  Error against 64 bits, activations N(0, 1) with 0.1% of
-// them 20 times larger: 1.5e-6 of the result (hi / lo bf16, before: 2.5e-6).
+// 32-element block becomes four E2M3 digits, each under its own scale for the
+// block: the power of two that takes the largest of what the digits before it
+// left to at most 7.5.  x - sum of digits is then within 2^-20 of the power of
+// two above the block's largest element (2^-19 of that element), and 2^-22 of
+// the element in the root mean square of normal activations.  The scales are the
+// instruction's own block scales.
+// v_mfma_scale_f32_32x32x64_f8f6f4 with E2M3 operands multiplies two digits of
+// 32 elements at once (the digits are its two K halves, against the same codes
+// twice), so a block of a 32 x 32 tile is two MFMAs, half of the f16 form's
+// four, folded into the f32 accumulators by one FMA per output with the
+// block's scale.
+//
+// That step is absolute within a block: beside an element much larger than the
+// rest, the rest lose bits, which shows in the outputs whose codes are small
+// there (a channel large in every row, with small weights).  So a row whose
+// blocks' squared maxima average kSpread times its mean magnitude squared (both as
+// exponents) gets four more digits in the blocks kFar binades above that
+// mean; the GEMM adds those blocks' products after its main loop.  Relative to
+// the result, K = 4096, against 64 bits: N(0, 1) 5.3e-7, with 0.1% of the elements 20
+// times larger 6.7e-7 (hi / lo bf16: 2.4e-6 both); two channels at 1000 and
+// codes of zero there 5.2e-7 (bf16 2.5e-6, four digits alone 1.5e-5); the worst
+// of some forty sets, with outliers just below the limits, 1.7e-6.  (Elements
+// 2^-23 of their block's largest and below keep 15 bits or more, as an f32
+// largest takes up to five of the eight digits.)
 //
 // What bounds it: VALU issue and MFMA power (16 fold FMAs and two MFMAs of 32
 // cycles per tile and block).  Weights are re-encoded once per call (0.875
 // bytes a weight, 18 us for 14336 x 4096, in the launch that encodes the
 // activations), which decoding in the GEMM would repeat for every 128 or 256
 // rows of x.  q4_0, N = 14336, K = 4096: M = 512 139 -> 106 us, M = 2048
-// 552 -> 328 us.
+// 552 -> 330 us (with blocks of eight digits: a third of them 125 and 444 us,
+// all 210 and 713).
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -45,7 +61,9 @@ typedef float f32x32 __attribute__((ext_vector_type(32)));
 // Activations of one 32-row m-tile and block: operands j = 0, 1 as
 // [64 lanes][16 B] then [64 lanes][8 B] (lane l: row l & 31, digit
 // 2 j + (l >> 5): 32 6-bit codes), then the block's scale bytes [64 lanes]
-// {operand 0, operand 1, 0, 0}.
+// {operand 0, operand 1, 0, 0}.  A second array of the same layout holds the
+// further digits of the blocks that have them, with a byte per eight rows and
+// block that says so, and one per eight rows (any block).
 constexpr int kXOp = 1536;
 constexpr int kXFrag = 2 * kXOp;
 constexpr int kXBlock = kXFrag + 256;
@@ -53,6 +71,11 @@ constexpr int kXBlock = kXFrag + 256;
 // codes, [32 rows] f32 scales.
 constexpr int kWBlock = 32 * 28;
 constexpr int kWSlot = 1024;                // its bytes in LDS (one load; the last 128 unused)
+// Rows and blocks with further digits (modelled over forty distributions:
+// silu(a) b and relu(a)^2 of normal a, b, whose ratio is 340-410, stay below;
+// with up to 800 the four digits' error is at most 1.7e-6 of any outputs).
+constexpr float kSpread = 800.0f;
+constexpr float kFar = 5.0f;
 
 // Codes 2 i and 2 i + 1 of a block's 32 are elements i and i + 16: the order
 // of the q4_0 bytes' nibbles, and of v_cvt_scalef32_2xpk16_fp6_f32.
@@ -76,12 +99,14 @@ __device__ __forceinline__ void byte_codes(uint32_t c, uint32_t& lo, uint32_t& h
 
 // One launch prepares both operands.  Workgroups [0, xwgs): eight activation
 // rows each and one of `slices` slices of K: the rows' power-of-two scales
-// (largest element in [0.5, 1)), then the digits of the slice's blocks, one
-// lane per row and block.  The next wwgs: weights, a wave per n-tile and eight
+// (largest element in [0.5, 1)) and spreads, then the digits of the slice's
+// blocks, one lane per row and block.  The next wwgs: weights, a wave per n-tile and eight
 // block pairs, one lane per row and pair.  Any beyond clear y.
 __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int M, int K,
                                                int slices, int blocks_per_slice, int xwgs,
-                                               uint8_t* __restrict__ xf, int* __restrict__ rexp,
+                                               uint8_t* __restrict__ xf, uint8_t* __restrict__ xr,
+                                               uint8_t* __restrict__ xflag,
+                                               uint8_t* __restrict__ xspread, int* __restrict__ rexp,
                                                const uint8_t* __restrict__ W, int N,
                                                uint8_t* __restrict__ wf, int wwgs,
                                                float* zero_y, long long ldy) {
@@ -135,22 +160,44 @@ __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int 
     return;
   }
 
-  __shared__ int sexp[8];
+  __shared__ int sexp[8], sfar[8];
   const int group = blockIdx.x / slices, slice = blockIdx.x % slices;
   const int m0 = 8 * group;
   const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  if (m0 + wave < M) {                             // wave w: the maximum of row m0 + w
-    const float* xr = x + static_cast<long long>(m0 + wave) * K;
+  if (m0 + wave < M) {                             // wave w: row m0 + w
+    const float* xr0 = x + static_cast<long long>(m0 + wave) * K;
     float mx = 0.f, z = 0.f;
-    auto see = [&](const f32x4& v) {
+    // exponents of the row's nonzero elements (sum and count); sum of 4^exponent
+    // of its nonzero blocks' maxima, as bs * 4^be, and their count
+    int esum = 0, count = 0, blocks = 0, be = -1000;
+    float bs = 0.f;
+    // v: this lane's elements of a block of 8 lanes (wide: of 32)
+    auto see = [&](const f32x4& v, bool wide) {
+      float bm = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        mx = fmaxf(mx, fabsf(v[e]));
+        const float a = fabsf(v[e]);
+        esum += __builtin_amdgcn_frexp_expf(a);   // 0 for 0
+        count += a > 0.f ? 1 : 0;
+        bm = fmaxf(bm, a);
         z = fmaf(0.0f, v[e], z);                   // NaN once an element is not finite
+      }
+      bm = group8_max(bm);
+      if (wide) {
+        bm = fmaxf(bm, __shfl_xor(bm, 8));
+        bm = fmaxf(bm, __shfl_xor(bm, 16));
+      }
+      mx = fmaxf(mx, bm);
+      if (bm > 0.f) {
+        const int ex = __builtin_amdgcn_frexp_expf(bm);
+        const int ne = max(be, ex);
+        bs = ldexpf(bs, 2 * (be - ne)) + ldexpf(1.0f, 2 * (ex - ne));
+        be = ne;
+        ++blocks;
       }
     };
     if (aligned) {
-      const f32x4* x4 = reinterpret_cast<const f32x4*>(xr);
+      const f32x4* x4 = reinterpret_cast<const f32x4*>(xr0);
       const int n4 = K / 4;
       int i = lane;
       for (; i + 448 < n4; i += 512) {
@@ -158,18 +205,24 @@ __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int 
 #pragma unroll
         for (int u = 0; u < 8; ++u) v[u] = x4[i + 64 * u];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) see(v[u]);
+        for (int u = 0; u < 8; ++u) see(v[u], false);
       }
-      for (; i < n4; i += 64) see(x4[i]);
+      for (; i < n4; i += 64) see(x4[i], false);
     } else {
-      for (int i = lane; i < K; i += 64) see(f32x4{xr[i], 0.f, 0.f, 0.f});
+      for (int i = lane; i < K; i += 64) see(f32x4{xr0[i], 0.f, 0.f, 0.f}, true);
     }
     mx = wave_max_nonneg(mx);
     const bool bad = __any(z != 0.0f);
     int e = 0;
     if (mx > 0.f && mx <= 3.402823466e38f) (void)frexpf(mx, &e);
+    // every lane of a block carries its term: the copies cancel in the ratio
+    const float sum = wave_sum(ldexpf(bs, max(2 * (be - e), -400)));
+    const float mean = wave_sum(static_cast<float>(esum)) / wave_sum(static_cast<float>(count));
+    const bool far = !bad && sum > kSpread * wave_sum(static_cast<float>(blocks)) *
+                                          exp2f(2.0f * (mean - static_cast<float>(e)));
     if (lane == 0) {
       sexp[wave] = bad ? 0 : e;
+      sfar[wave] = far ? static_cast<int>(ceilf(mean + kFar)) - e : INT_MAX;
       if (slice == 0) rexp[m0 + wave] = bad ? kRowNonfinite : e;
     }
   }
@@ -177,7 +230,9 @@ __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int 
   const int row = lane & 7;
   const int m = m0 + row;
   if (m >= M) return;
-  const int e = -sexp[row];
+  const bool spread = __any(sfar[row] != INT_MAX);
+  if (slice == 0 && tid == 0) xspread[group] = spread ? 1 : 0;
+  const int e = -sexp[row], farex = sfar[row];
   const int b0 = slice * blocks_per_slice, b1 = min(b0 + blocks_per_slice, nb);
   for (int b = b0 + 8 * wave + (lane >> 3); b < b1; b += 64) {
     const float* src = x + static_cast<long long>(m) * K + 32 * b;
@@ -200,45 +255,56 @@ __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int 
         hi[i] = src[16 + i];
       }
     }
-    float mx = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       lo[i] = ldexpf(lo[i], e);
       hi[i] = ldexpf(hi[i], e);
-      mx = fmaxf(mx, fmaxf(fabsf(lo[i]), fabsf(hi[i])));
     }
-    // Digit t of an element is its E2M3 code at scale 2^(ex - 2 - 5 t): the
-    // first is at most 4 in magnitude, and each leaves at most 2^-5 of the
-    // largest digit for the next (exactly: the remainder is representable).
-    // Blocks below 2^-100 of the row's largest element share that scale.
-    int ex = -100;
-    if (mx > 0.f && mx <= 3.402823466e38f) (void)frexpf(mx, &ex);
-    ex = ex < -100 ? -100 : ex;
-    uint8_t* d = xf + (static_cast<long long>(m >> 5) * nb + b) * kXBlock;
+    // Four digits of what lo, hi hold (which keep what the digits leave,
+    // exactly) to a block's fragments at d; the exponent of the largest.
     const int r = m & 31;
+    auto digits = [&](uint8_t* d) {
+      int first = INT_MIN;
+      uint32_t sb[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float scale = __int_as_float((ex - 2 - 5 * t + 127) << 23);
-      const u32x6 o = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo, hi, scale);
-      if (t < 3) {
-        const f32x32 f = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(o, scale);
+      for (int t = 0; t < 4; ++t) {
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fmaxf(fabsf(lo[i]), fabsf(hi[i])));
+        int ex = -123;
+        float f = 0.f;
+        if (mx > 0.f && mx <= 3.402823466e38f) {
+          f = frexpf(mx, &ex);
+          if (t == 0) first = ex;
+        }
+        // 2^s: the largest at most 7.5 of it
+        const int s = max(ex - (f > 0.9375f ? 2 : 3), -126);
+        const float scale = __int_as_float((s + 127) << 23);
+        const u32x6 o = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo, hi, scale);
+        const f32x32 v = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(o, scale);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          lo[i] -= f[2 * i];
-          hi[i] -= f[2 * i + 1];
+          lo[i] -= v[2 * i];
+          hi[i] -= v[2 * i + 1];
         }
+        uint8_t* op = d + (t >> 1) * kXOp;
+        const int l = r + 32 * (t & 1);
+        *reinterpret_cast<u32x4*>(op + 16 * l) = u32x4{o[0], o[1], o[2], o[3]};
+        *reinterpret_cast<u32x2*>(op + 1024 + 8 * l) = u32x2{o[4], o[5]};
+        sb[t] = static_cast<uint32_t>(s + 127);
       }
-      uint8_t* op = d + (t >> 1) * kXOp;
-      const int l = r + 32 * (t & 1);
-      *reinterpret_cast<u32x4*>(op + 16 * l) = u32x4{o[0], o[1], o[2], o[3]};
-      *reinterpret_cast<u32x2*>(op + 1024 + 8 * l) = u32x2{o[4], o[5]};
-    }
-    // scale bytes (exponent + 127) of digits h and 2 + h, h = 0, 1
+      // scale bytes (exponent + 127) of digits h and 2 + h, h = 0, 1
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t s0 = static_cast<uint32_t>(ex - 2 - 5 * h + 127);
-      *reinterpret_cast<uint32_t*>(d + kXFrag + 4 * (r + 32 * h)) = s0 | ((s0 - 10) << 8);
-    }
+      for (int h = 0; h < 2; ++h)
+        *reinterpret_cast<uint32_t*>(d + kXFrag + 4 * (r + 32 * h)) = sb[h] | (sb[2 + h] << 8);
+      return first;
+    };
+    const long long at = static_cast<long long>(m >> 5) * nb + b;
+    const bool more = digits(xf + at * kXBlock) >= farex;
+    // further digits for all eight rows once one of them needs them
+    const bool any = (__ballot(more) >> (lane & 56) & 0xFFu) != 0;
+    if (row == 0) xflag[4 * at + (r >> 3)] = any ? 1 : 0;
+    if (any) (void)digits(xr + at * kXBlock);
   }
 }
 
@@ -261,9 +327,10 @@ struct Mx {
 
 template <int TM, int TN, int WGM, int WGN, int S>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void mx_gemm(
-    const uint8_t* __restrict__ wf, const uint8_t* __restrict__ xf, float* __restrict__ y,
-    const int* __restrict__ rexp, const uint8_t* __restrict__ W, const float* __restrict__ x, int M,
-    int N, long long ldy, int K, int mblocks, int nblocks, int blocks_per_split, int ks_count) {
+    const uint8_t* __restrict__ wf, const uint8_t* __restrict__ xf, const uint8_t* __restrict__ xr,
+    const uint8_t* __restrict__ xflag, const uint8_t* __restrict__ xspread, float* __restrict__ y,
+    const int* __restrict__ rexp, const uint8_t* __restrict__ W, const float* __restrict__ x, int M, int N, long long ldy,
+    int K, int mblocks, int nblocks, int blocks_per_split, int ks_count) {
   using C = Mx<TM, TN, WGM, WGN, S>;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[C::lds];
   const int tid = threadIdx.x;
@@ -359,6 +426,17 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void mx_gemm(
     d = *reinterpret_cast<const float*>(p + 768 + 4 * col);
   };
 
+  // Per m-tile a byte for each eight rows: any of them with further digits at
+  // all, and (per block) in block b.  Bytes past M are not set.
+  auto in_rows = [&](int tm, uint32_t f) {
+    const int groups = (M - 32 * (mt0 + wm * TM + tm) + 7) / 8;
+    return groups >= 4 ? f : groups <= 0 ? 0u : f & ((1u << (8 * groups)) - 1);
+  };
+  uint32_t further = 0;
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm)
+    further |= in_rows(tm, reinterpret_cast<const uint32_t*>(xspread)[mt0 + wm * TM + tm]);
+
   if (steps > 0) {
     // Barrier B_s stands before the last m-tile of step s.  Step s issues,
     // before B_s, stage s + S - 1 into the slot of stage s - 1; at B_s the
@@ -443,6 +521,60 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void mx_gemm(
   }
   wait_vmcnt<0>();   // no global->LDS load may outlive the workgroup's LDS
 
+  // The further digits, from memory: few blocks, each wave its own m-tiles'.
+  if (further != 0) {
+    for (int c0 = b0; c0 < b1; c0 += 64) {
+      uint32_t f[TM];
+      uint64_t todo = 0;
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) {
+        const int b = min(c0 + lane, b1 - 1);
+        const long long at = static_cast<long long>(mt0 + wm * TM + tm) * nb + b;
+        f[tm] = c0 + lane < b1 ? in_rows(tm, reinterpret_cast<const uint32_t*>(xflag)[at]) : 0;
+        todo |= __ballot(f[tm] != 0);
+      }
+      while (todo != 0) {
+        const int i = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        i32x8 w[TN], a[TM][2];
+        int sc[TM];
+        float d[TN];
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) {
+          const uint8_t* p = wf + min(nt0 + wn * TN + tn, ntiles - 1) * wtile + (c0 + i) * kWBlock;
+          read6(p + 16 * col, p + 512 + 8 * col, w[tn]);
+          d[tn] = *reinterpret_cast<const float*>(p + 768 + 4 * col);
+        }
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const uint32_t g = __builtin_amdgcn_readlane(f[tm], i);
+          const i32x8 zero = {};
+          a[tm][0] = a[tm][1] = zero;
+          sc[tm] = 0;
+          if (g >> (8 * (col >> 3)) & 0xFF) {
+            const uint8_t* p = xr + (mt0 + wm * TM + tm) * xtile + (c0 + i) * kXBlock;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              read6(p + j * kXOp + 16 * lane, p + j * kXOp + 1024 + 8 * lane, a[tm][j]);
+            sc[tm] = *reinterpret_cast<const int*>(p + kXFrag + 4 * lane);
+          }
+        }
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) {
+            const f32x16 z = {};
+            f32x16 v = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[tm][0], w[tn], z, 2, 2, 0,
+                                                                       sc[tm], 0, 130);
+            v = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[tm][1], w[tn], v, 2, 2, 1, sc[tm],
+                                                                0, 130);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[tm][tn][e] = fmaf(v[e], d[tn], acc[tm][tn][e]);
+          }
+      }
+    }
+  }
+
   store_tiles<TM, TN>(acc, rexp, y, ldy, ks_count > 1, 32 * (mt0 + wm * TM), 32 * (nt0 + wn * TN), M, N,
                       [&](int m, int n) {
                         return nonfinite_blocks_f32<kQ4_0>(W + static_cast<long long>(n) * nb * 18,
@@ -457,51 +589,45 @@ constexpr int kTiles = 3;
 constexpr Tile kTile[kTiles] = {
     {256, 256, 1, 0.88, 1.30}, {128, 256, 1, 0.42, 0.74}, {128, 128, 2, 0.35, 0.80}};
 
+// A call's operands: activation fragments, their further digits and which blocks
+// have them, row exponents, re-encoded weights.
+struct Operands {
+  uint8_t *xf, *xr, *xflag, *xspread, *wf;
+  int* rexp;
+};
+
 template <int TM, int TN, int WGM, int WGN, int S>
-hipError_t launch_tile(const uint8_t* wf, const uint8_t* xf, float* y, const int* rexp,
-                       const uint8_t* W, const float* x, int m, int n, long long ldy, int k,
-                       const TilePlan& p, hipStream_t s) {
+hipError_t launch_tile(const Operands& o, float* y, const uint8_t* W, const float* x, int m, int n,
+                       long long ldy, int k, const TilePlan& p, hipStream_t s) {
   using C = Mx<TM, TN, WGM, WGN, S>;
   const int mblocks = (m + C::BM - 1) / C::BM, nblocks = (n + C::BN - 1) / C::BN;
   mx_gemm<TM, TN, WGM, WGN, S><<<static_cast<unsigned>(mblocks) * nblocks * p.ks, 64 * C::NW, 0, s>>>(
-      wf, xf, y, rexp, W, x, m, n, ldy, k, mblocks, nblocks, p.per, p.ks);
+      o.wf, o.xf, o.xr, o.xflag, o.xspread, y, o.rexp, W, x, m, n, ldy, k, mblocks, nblocks, p.per, p.ks);
   return hipGetLastError();
 }
 
-// One chunk of at most kRows activation rows and as many weight rows as their
-// re-encoded form allows.
-hipError_t run_mx(const uint8_t* W, const float* x, float* y, int m, int n, long long ldy, int k,
-                  hipStream_t s, StreamWorkspace* ws) {
+// One chunk of rows and one of weight rows.
+hipError_t run_mx(const Operands& o, const uint8_t* W, const float* x, float* y, int m, int n,
+                  long long ldy, int k, hipStream_t s) {
   const int nb = k / 32;
   const TilePlan p = plan_tiles(kTile, kTiles, m, n, nb, device_cu_count(), 0, 2);
-  const size_t xf_bytes = static_cast<size_t>((m + 255) / 256 * 8) * nb * kXBlock;
-  const size_t wf_bytes = static_cast<size_t>((n + 31) / 32) * nb * kWBlock + 128;   // kWSlot reads
-  void* buf = nullptr;
-  hipError_t e = stream_buffer(ws, s, xf_bytes + wf_bytes, 0, &buf);
-  if (e != hipSuccess) return e;
-  uint8_t* xf = static_cast<uint8_t*>(buf);
-  uint8_t* wf = xf + xf_bytes;
-  // read in whole tiles: padded to the largest
-  e = stream_buffer(ws, s, sizeof(int) * static_cast<size_t>((m + 255) / 256 * 256), 1, &buf);
-  if (e != hipSuccess) return e;
-  int* rexp = static_cast<int*>(buf);
-
   // activations: eight rows a workgroup, K in as many slices as give ~512
   // workgroups of at least 64 blocks (one per eight lanes)
   const int groups = (m + 7) / 8;
   const int want = std::max(1, std::min((nb + 63) / 64, 512 / groups));
   const int per_slice = (nb + want - 1) / want;
   const int slices = (nb + per_slice - 1) / per_slice;
+  const int xwgs = groups * slices;
   const long long items = static_cast<long long>((n + 31) / 32) * ((k / 64 + 7) / 8);
-  const long long clear = p.ks == 2 ? 512 : 0;
-  mx_prep<<<static_cast<unsigned>(groups * slices + (items + 7) / 8 + clear), 512, 0, s>>>(
-      x, m, k, slices, per_slice, groups * slices, xf, rexp, W, n, wf,
-      static_cast<int>((items + 7) / 8), y, ldy);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  const int wwgs = static_cast<int>((items + 7) / 8);
+  mx_prep<<<static_cast<unsigned>(xwgs) + wwgs + (p.ks == 2 ? 512 : 0), 512, 0, s>>>(
+      x, m, k, slices, per_slice, xwgs, o.xf, o.xr, o.xflag, o.xspread, o.rexp, W, n, o.wf, wwgs, y, ldy);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
   switch (p.tile) {
-    case 0: return launch_tile<4, 2, 2, 4, 4>(wf, xf, y, rexp, W, x, m, n, ldy, k, p, s);
-    case 1: return launch_tile<2, 2, 2, 4, 6>(wf, xf, y, rexp, W, x, m, n, ldy, k, p, s);
-    default: return launch_tile<2, 2, 2, 2, 4>(wf, xf, y, rexp, W, x, m, n, ldy, k, p, s);
+    case 0: return launch_tile<4, 2, 2, 4, 4>(o, y, W, x, m, n, ldy, k, p, s);
+    case 1: return launch_tile<2, 2, 2, 4, 6>(o, y, W, x, m, n, ldy, k, p, s);
+    default: return launch_tile<2, 2, 2, 2, 4>(o, y, W, x, m, n, ldy, k, p, s);
   }
 }
 
@@ -517,18 +643,33 @@ bool mx_pays(int m, int n) { return m >= 384 && n >= 2048; }
 hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n, int k,
                            hipStream_t s, StreamWorkspace* ws) {
   const auto* w = static_cast<const uint8_t*>(W);
-  // Activation rows in chunks whose digits (3.25 bytes an element) take at
+  const int nb = k / 32;
+  // Activation rows in chunks whose digits (twice 3.25 bytes an element) take at
   // most 256 MB, weight rows in chunks of at most 256 MB (0.875 bytes a weight).
-  const long long fit = (256LL << 20) / (4LL * k) / 256 * 256;
+  const long long fit = (256LL << 20) / (7LL * k) / 256 * 256;
   const int mchunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, INT_MAX / 2)));
   const long long nfit = (256LL << 20) / k / 256 * 256;
   const int nchunk = static_cast<int>(std::max<long long>(256, std::min<long long>(nfit, INT_MAX / 2)));
+  const size_t mpad = (std::min(m, mchunk) + 255) / 256 * 256;   // read in whole tiles
+  const size_t xf_bytes = mpad / 32 * nb * kXBlock, flag_bytes = mpad / 8 * (nb + 1);
+  const size_t wf_bytes = static_cast<size_t>((std::min(n, nchunk) + 31) / 32) * nb * kWBlock + 128;   // kWSlot reads
+  void* buf = nullptr;
+  hipError_t e = stream_buffer(ws, s, 2 * xf_bytes + flag_bytes + wf_bytes, 0, &buf);
+  if (e != hipSuccess) return e;
+  Operands o;
+  o.xf = static_cast<uint8_t*>(buf);
+  o.xr = o.xf + xf_bytes;
+  o.xflag = o.xr + xf_bytes;
+  o.xspread = o.xflag + mpad / 8 * nb;
+  o.wf = o.xflag + flag_bytes;
+  e = stream_buffer(ws, s, sizeof(int) * mpad, 1, &buf);
+  if (e != hipSuccess) return e;
+  o.rexp = static_cast<int*>(buf);
   for (int m0 = 0; m0 < m; m0 += mchunk)
     for (int n0 = 0; n0 < n; n0 += nchunk) {
-      const hipError_t e = run_mx(w + static_cast<long long>(n0) * (k / 32) * 18,
-                                  x + static_cast<long long>(m0) * k,
-                                  y + static_cast<long long>(m0) * n + n0, std::min(mchunk, m - m0),
-                                  std::min(nchunk, n - n0), n, k, s, ws);
+      e = run_mx(o, w + static_cast<long long>(n0) * nb * 18,
+                 x + static_cast<long long>(m0) * k, y + static_cast<long long>(m0) * n + n0,
+                 std::min(mchunk, m - m0), std::min(nchunk, n - n0), n, k, s);
       if (e != hipSuccess) return e;
     }
   return hipSuccess;

@@ -6,8 +6,9 @@
 // 234-286): y[m][n] = sum_b d[n][b] * sum_{k in b} q[n][k] * x[m][k].
 //
 // Numerics.  Each activation row is scaled by a power of two and split into
-// hi = f16(x) and lo = f16(x - hi), so x - hi - lo is within 2^-22 |x|; codes
-// (-128..127) are exact in f16.  A 32-element block of a 32 x 32 tile is four
+// hi = f16(x) and lo = f16(x - hi), so x - hi - lo is within 2^-22 |x| + 2^-25
+// at that scale (largest element in [2^14, 2^15)); codes (-128..127) are exact
+// in f16.  A 32-element block of a 32 x 32 tile is four
 // v_mfma_f32_32x32x16_f16 (two K halves, hi and lo) into a zeroed tile, folded
 // into the f32 accumulators by one FMA per output with the block's scale.
 //
