@@ -6,11 +6,11 @@
 // Numerics.  Activation rows are scaled by a power of two so that their
 // largest element lies in [2^14, 2^15).  f16 and bf16 activations are then f16
 // values (exactly, down to 2^-28 of the row's largest), f32 ones a pair hi + lo
-// of them within 2^-22 of each element.  Codes minus an integral zero point
-// (|q - z| <= 1280) are exact in f16, products and sums are f32.  A zero point
-// that is not an integer in [-1152, 896] stays out of the codes: its product
-// with the sum of x, taken by MFMAs against a column of ones, is subtracted in
-// f32.  An f32 row holding 16-bit values has lo = 0 throughout and gives the
+// of them within 2^-22 of each element.  Codes minus the integer of [-1152, 896]
+// next to their zero point (at most 1280 in magnitude) are exact in f16,
+// products and sums are f32.  What of the zero point that leaves (up to 0.5 of a
+// fractional one) times the sum of x is subtracted in f32, so nothing is summed
+// that is larger than the codes' distances from their zero point.  An f32 row holding 16-bit values has lo = 0 throughout and gives the
 // bits of the 16-bit call.
 //
 // What bounds it: with few workgroups the chain of a step (one barrier, the
@@ -19,7 +19,9 @@
 // shared by the wave's m-tiles, and with groups the fold, one FMA per output and
 // 64 columns) and the operands' way into LDS.  K = 4096, groups of 32, N =
 // 14336, M = 512: 586 us on the row planes -> 151; groups of 128 257 -> 120; row
-// scales N = 4096 63 -> 41 (16-bit activations).  Small tiles with rings of 6-8
+// scales N = 4096 63 -> 41 (16-bit activations).  Fractional zero points: groups
+// of 128, M = 512 257 on the planes, 200 with MFMAs over all of x against ones,
+// 146 with the sums that the prep writes.  Small tiles with rings of 6-8
 // stages while the larger leave CUs idle; 128 x 256 above that.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -50,13 +52,16 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSlotBytes = 1024;
 
 // Eight activation rows per workgroup, K in gridDim.y slices of whole steps:
-// the rows' scales (over whole rows, in every slice), then the fragments.
+// the rows' scales (over whole rows, in every slice), then the fragments, and
+// (sums = 1, 2) each row's scaled sum over every 64 or 32 columns, as
+// xs[32-row m-tile][K / 64 * sums][32].
 // Each 128-byte line is eight rows' 16-byte pieces, stored at once.
 template <int P>
 __global__ __launch_bounds__(512) void f16_prep(const void* __restrict__ x, int xtype,
                                                 long long ldx, bool vec, int M, int K,
                                                 int steps_per_slice, uint8_t* __restrict__ xf,
-                                                int* __restrict__ rexp) {
+                                                int* __restrict__ rexp, float* __restrict__ xs,
+                                                int sums) {
   __shared__ int sexp[8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m0 = 8 * blockIdx.x;
@@ -119,15 +124,25 @@ __global__ __launch_bounds__(512) void f16_prep(const void* __restrict__ x, int 
     float v[8];
     load8(src + 64LL * t, v);
     f16x8 hi, lo;
+    float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const float w = ldexpf(v[i], e);
+      sum += w;
       hi[i] = static_cast<_Float16>(w);
       if constexpr (P == 2) lo[i] = static_cast<_Float16>(w - static_cast<float>(hi[i]));
     }
     uint8_t* d = dst + static_cast<long long>(t) * (4 * P * kSlotBytes);
     *reinterpret_cast<f16x8*>(d) = hi;
     if constexpr (P == 2) *reinterpret_cast<f16x8*>(d + kSlotBytes) = lo;
+    if (sums > 0) {
+      sum += __shfl_xor(sum, 8);
+      sum += __shfl_xor(sum, 32);
+      if (sums == 1) sum += __shfl_xor(sum, 16);
+      if (lane < 16 * sums && s == 0)
+        xs[(static_cast<long long>(m >> 5) * steps * sums + t * sums + (sums == 2 ? b : 0)) * 32 +
+           (m & 31)] = sum;
+    }
   }
 }
 
@@ -150,9 +165,9 @@ __device__ __forceinline__ T* pick(T* a, T* b, bool second) {
   return reinterpret_cast<T*>(x ^ ((x ^ y) & (0 - static_cast<uint64_t>(second))));
 }
 
-// An integral zero point that codes can be reduced by exactly in f16.
-__device__ __forceinline__ bool code_zero(float z) {
-  return z >= -1152.0f && z <= 896.0f && z == rintf(z);
+// The part of a zero point that codes can be reduced by exactly in f16.
+__device__ __forceinline__ float code_zero(float z) {
+  return fminf(fmaxf(rintf(z), -1152.0f), 896.0f);
 }
 
 // The projection of activation row xr (elements) on weight row n in the
@@ -191,7 +206,7 @@ struct F16Tile {
 template <int P, int TM, int TN, int WGM, int WGN, int S, int GPS, bool SWIGLU>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
     const uint8_t* __restrict__ xf, const F16Out o, const int* __restrict__ rexp,
-    const void* __restrict__ x, int xtype, long long ldx, int M, int K, int mblocks,
+    const float* __restrict__ xs, const void* __restrict__ x, int xtype, long long ldx, int M, int K, int mblocks,
     int nblocks) {
   using C = F16Tile<P, TM, TN, WGM, WGN, S, GPS>;
   static_assert(!SWIGLU || TN == 2, "gate and up tiles side by side");
@@ -288,8 +303,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.f;
 
-  // One step's weight operands: f16 codes less their zero points (those that
-  // are code_zero; `rest` notes any other), and each group's scale.
+  // One step's weight operands: f16 codes less their zero points' code_zero
+  // (`rest` notes any that leave something), and each group's scale.
   constexpr int NG = GPS > 0 ? GPS : 1;
   struct Weights {
     f16x8 w[TN][4];
@@ -304,8 +319,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
       bool second;
       const int n = row_of((wn * TN + tn) * 32 + col, second);
       const float z = pick(o.zero[0], o.zero[1], second)[n];
-      rz[tn] = code_zero(z) ? z : 0.f;
-      rest = rest || !code_zero(z);
+      rz[tn] = code_zero(z);
+      rest = rest || rz[tn] != z;
     }
   }
   struct Raw {
@@ -335,9 +350,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
       for (int g = 0; g < NG; ++g) {
         if constexpr (GPS > 0) {
           o2.s[tn][g] = r.sz[tn][g].x;
-          const bool in = code_zero(r.sz[tn][g].y);
-          z[g] = zeros && in ? r.sz[tn][g].y : 0.f;
-          rest = rest || (zeros && !in);
+          z[g] = zeros ? code_zero(r.sz[tn][g].y) : 0.f;
+          rest = rest || (zeros && z[g] != r.sz[tn][g].y);
         } else {
           z[g] = rz[tn];
         }
@@ -427,41 +441,47 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
   }
   wait_vmcnt<0>();   // no global->LDS load may outlive the workgroup's LDS
 
-  // Zero points beyond the codes' reach: each step's sums of x (MFMAs against
-  // ones), times them, from a second pass over the activations.
+  // What the codes left of the zero points: the product of the rows' sums of x
+  // over a group (row scales: a step) with it and the scale, two of them an f32
+  // MFMA.
   if (__any(rest)) {
-    const _Float16 one = static_cast<_Float16>(1.0f);
-    const f16x8 ones = f16x8{one, one, one, one, one, one, one, one};
-#pragma unroll 1
-    for (int t = 0; t < steps; ++t) {
+    const int per = GPS == 1 ? o.gsize / 64 : 1;   // sums to a group
+    const int cols = GPS == 1 ? o.groups : NG * steps;
+    constexpr int U = 4;                           // MFMAs whose operands load together
+    for (int c0 = 0; c0 < cols; c0 += 2 * U) {
+      float f[U][TN], a[U][TM];
 #pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        float f[TN];
+      for (int u = 0; u < U; ++u) {
+        const int c = min(c0 + 2 * u + half, cols - 1);
+        const bool in = c0 + 2 * u + half < cols;
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) {
           bool second;
           const long long n = row_of((wn * TN + tn) * 32 + col, second);
-          const long long si = n * o.groups + (GPS == 0 ? 0 : (64 * t + 32 * g) / o.gsize);
+          const long long si = n * o.groups + (GPS == 0 ? 0 : c);
           const float z = pick(o.zero[0], o.zero[1], second)[si];
           const float sc = GPS == 0 ? 1.0f : pick(o.scale[0], o.scale[1], second)[si];
-          f[tn] = code_zero(z) ? 0.f : -z * sc;
+          f[u][tn] = in ? (code_zero(z) - z) * sc : 0.f;
         }
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const uint8_t* a = xf + (mt0 + wm * TM + tm) * xtile +
-                             static_cast<long long>(t) * XT * kSlotBytes + 16 * lane;
-          f32x16 c = {};
+        for (int tm = 0; tm < TM; ++tm) a[u][tm] = 0.f;
+      }
+      for (int j = 0; j < per; ++j)
 #pragma unroll
-          for (int q = XT / NG * g; q < XT / NG * (g + 1); ++q)
-            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                *reinterpret_cast<const f16x8*>(a + q * kSlotBytes), ones, c, 0, 0, 0);
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm) {
+            const long long c = static_cast<long long>(mt0 + wm * TM + tm) * cols + c0 + 2 * u + half;
+            const float v = xs[(min(c, (mt0 + wm * TM + tm + 1LL) * cols - 1) * per + j) * 32 + col];
+            a[u][tm] += c0 + 2 * u + half < cols ? v : 0.f;
+          }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
           for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-              if (f[tn] != 0.f) acc[tm][tn][e] = fmaf(c[e], f[tn], acc[tm][tn][e]);
-        }
-      }
+            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][tm], f[u][tn], acc[tm][tn], 0, 0, 0);
     }
   }
 
@@ -507,26 +527,26 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void f16_gemm(
 }
 
 template <int P, int TM, int TN, int WGM, int WGN, int S, int GPS, bool SWIGLU>
-hipError_t launch_tile(const uint8_t* xf, const F16Out& o, const int* rexp, const void* x, int xtype,
-                       long long ldx, int m, int k, hipStream_t s) {
+hipError_t launch_tile(const uint8_t* xf, const F16Out& o, const int* rexp, const float* xs,
+                       const void* x, int xtype, long long ldx, int m, int k, hipStream_t s) {
   using C = F16Tile<P, TM, TN, WGM, WGN, S, GPS>;
   const int mblocks = (m + C::BM - 1) / C::BM;
   const int bn = SWIGLU ? C::BN / 2 : C::BN;
   const int nblocks = (o.rows + bn - 1) / bn;
   f16_gemm<P, TM, TN, WGM, WGN, S, GPS, SWIGLU>
-      <<<static_cast<unsigned>(mblocks) * nblocks, 64 * C::NW, 0, s>>>(xf, o, rexp, x, xtype, ldx, m,
-                                                                      k, mblocks, nblocks);
+      <<<static_cast<unsigned>(mblocks) * nblocks, 64 * C::NW, 0, s>>>(xf, o, rexp, xs, x, xtype, ldx,
+                                                                      m, k, mblocks, nblocks);
   return hipGetLastError();
 }
 
 // Tile by workgroups: the small one while the larger would leave CUs idle.
 template <int P, int GPS, bool SWIGLU>
-hipError_t launch_f16(const uint8_t* xf, const F16Out& o, const int* rexp, const void* x, int xtype,
-                      long long ldx, int m, int k, hipStream_t s) {
+hipError_t launch_f16(const uint8_t* xf, const F16Out& o, const int* rexp, const float* xs,
+                      const void* x, int xtype, long long ldx, int m, int k, hipStream_t s) {
   const long long cols = SWIGLU ? 2LL * o.rows : o.rows;
   const long long big = ((m + 127) / 128) * ((cols + 127) / 128);
 #define QC_F16(TM_, TN_, A_, B_, S_) \
-  launch_tile<P, TM_, TN_, A_, B_, S_, GPS, SWIGLU>(xf, o, rexp, x, xtype, ldx, m, k, s)
+  launch_tile<P, TM_, TN_, A_, B_, S_, GPS, SWIGLU>(xf, o, rexp, xs, x, xtype, ldx, m, k, s)
   if (big >= 5 * device_cu_count() / 4) return QC_F16(2, 2, 2, 4, P == 2 ? 3 : GPS == 0 ? 5 : 4);
   if constexpr (SWIGLU) return QC_F16(1, 2, 2, 2, P == 1 ? 8 : 6);
   else return QC_F16(2, 1, 1, 4, P == 1 ? 8 : 6);
@@ -550,9 +570,15 @@ hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k,
   std::unique_lock<std::mutex> hold;
   uint8_t* base = nullptr;
   const size_t xf_bytes = up256(2ull * p * rows * k);
-  hipError_t e = call_scratch(s, xf_bytes + 4ull * rows, hold, reinterpret_cast<void**>(&base));
+  // zero points: the rows' sums over 32 (groups of 32) or 64 columns
+  bool zeros = false;
+  for (int i = 0; i < L.nw; ++i) zeros = zeros || sg.zero[i] != nullptr;
+  const int sums = !zeros ? 0 : gps == 2 ? 2 : 1;
+  hipError_t e = call_scratch(s, xf_bytes + 4ull * rows + 4ull * rows * (k / 64) * sums, hold,
+                              reinterpret_cast<void**>(&base));
   if (e != hipSuccess) return e;
   int* rexp = reinterpret_cast<int*>(base + xf_bytes);
+  float* xs = reinterpret_cast<float*>(rexp + rows);
   for (int m0 = 0; m0 < m; m0 += chunk) {
     const int mc = std::min(chunk, m - m0);
     const void* xc = static_cast<const uint8_t*>(L.x) + es * static_cast<size_t>(m0) * L.ldx;
@@ -560,8 +586,8 @@ hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k,
     const int want = std::max(1, std::min((steps + 7) / 8, 512 / groups));
     const int per = (steps + want - 1) / want;
     const dim3 grid(groups, (steps + per - 1) / per);
-    if (p == 2) f16_prep<2><<<grid, 512, 0, s>>>(xc, L.xtype, L.ldx, vec, mc, k, per, base, rexp);
-    else f16_prep<1><<<grid, 512, 0, s>>>(xc, L.xtype, L.ldx, vec, mc, k, per, base, rexp);
+    if (p == 2) f16_prep<2><<<grid, 512, 0, s>>>(xc, L.xtype, L.ldx, vec, mc, k, per, base, rexp, xs, sums);
+    else f16_prep<1><<<grid, 512, 0, s>>>(xc, L.xtype, L.ldx, vec, mc, k, per, base, rexp, xs, sums);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     for (int i = 0; i < nmat; ++i) {
       const bool pair = L.mode == 1;
@@ -572,7 +598,7 @@ hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k,
                      sg.ld[i], sg.ytype[i], static_cast<int>(L.w[i].rows), sg.bias, sg.act,
                      !pair && i == 0 && (sg.bias != nullptr || sg.act != 0) ? 1 : 0, sg.groups,
                      sg.gsize};
-#define QC_F16(P_, G_, W_) launch_f16<P_, G_, W_>(base, o, rexp, xc, L.xtype, L.ldx, mc, k, s)
+#define QC_F16(P_, G_, W_) launch_f16<P_, G_, W_>(base, o, rexp, xs, xc, L.xtype, L.ldx, mc, k, s)
 #define QC_F16_G(P_, W_) \
   gps == 0 ? QC_F16(P_, 0, W_) : gps == 1 ? QC_F16(P_, 1, W_) : QC_F16(P_, 2, W_)
       e = p == 2 ? (pair ? QC_F16_G(2, true) : QC_F16_G(2, false))

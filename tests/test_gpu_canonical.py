@@ -761,3 +761,37 @@ def test_cint8_f16_route_epilogue(qc, oracle, dev):
                                     activation=act) == 0
         v = ys[0].double().cpu().numpy() + bias.double().cpu().numpy()[None, :]
         assert np.allclose(y.cpu().numpy(), oracle.linear_activation_f64(v, act), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("m,rows,cols,gsize,storage", [
+    (65, 300, 4096, 128, 0), (200, 1000, 4096, 0, 0), (40, 200, 4096, 32, 0), (130, 257, 1024, 64, 0),
+    (300, 129, 8192, 256, 1), (33, 100, 16448, 0, 2), (70, 66, 64, 32, 0)])
+def test_cint8_f16_route_codes_near_zero_points(qc, dev, m, rows, cols, gsize, storage):
+    """Codes within 3.5 of fractional zero points and of ones past the codes: the
+    result is small against the codes' own products, so a zero point that is
+    taken off at the end of K would cost it bits.  Each product and sum is f32 of
+    values no larger than 4.5 |x| (or, past the codes, than the result's own):
+    sums of K / 32 <= 514 rounded terms are within sqrt(514) 2^-24 = 1.4e-6."""
+    import torch
+    print(f"cint8 near zero m={m} rows={rows} cols={cols} gsize={gsize} storage={storage}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m + cols)
+    groups = cols // gsize if gsize else 1
+    centre = torch.randint(-120, 120, (rows, groups), generator=g, device=dev)
+    z = centre.float() + torch.rand((rows, groups), generator=g, device=dev) - 0.5
+    z[::2] = centre[::2].float() + 0.5             # rounds to even codes
+    far = torch.arange(rows, device=dev) % 5 == 3
+    z[far] = centre[far].float() * 40.0 + 0.25     # partly past what codes are reduced by
+    step = torch.randint(-3, 4, (rows, groups, cols // groups), generator=g, device=dev)
+    codes = (centre[:, :, None] + step).to(torch.int8).reshape(rows, cols).contiguous()
+    scales = 1e-2 * (0.5 + torch.rand((rows, groups), generator=g, device=dev))
+    w = qc.cint8_weights(codes, scales, z, rows, cols, groups)
+    wd = ((codes.double().reshape(rows, groups, -1) - z.double()[:, :, None]) *
+          scales.double()[:, :, None]).reshape(rows, cols)
+    x = torch.randn((m, cols), generator=g, device=dev)
+    x = x if storage == 0 else x.half() if storage == 1 else x.bfloat16()
+    y = torch.full((m, rows), float("nan"), device=dev)
+    assert qc.cint8_project_raw(0, [w], x, storage, m, [y], [0]) == 0
+    torch.cuda.synchronize()
+    y64 = x.double() @ wd.T.contiguous()
+    err = (y.double() - y64).norm(dim=0) / y64.norm(dim=0)
+    assert float(err.max()) < 2e-6, float(err.max())
