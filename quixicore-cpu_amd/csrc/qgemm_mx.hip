@@ -606,9 +606,10 @@ hipError_t launch_tile(const Operands& o, float* y, const uint8_t* W, const floa
   return hipGetLastError();
 }
 
-// One chunk of rows and one of weight rows.
-hipError_t run_mx(const Operands& o, const uint8_t* W, const float* x, float* y, int m, int n,
-                  long long ldy, int k, hipStream_t s) {
+// One chunk of rows and one of weight rows, each encoded here unless a call
+// before did.
+hipError_t run_mx(const Operands& o, bool encode_x, bool encode_w, const uint8_t* W, const float* x,
+                  float* y, int m, int n, long long ldy, int k, hipStream_t s) {
   const int nb = k / 32;
   const TilePlan p = plan_tiles(kTile, kTiles, m, n, nb, device_cu_count(), 0, 2);
   // activations: eight rows a workgroup, K in as many slices as give ~512
@@ -617,18 +618,28 @@ hipError_t run_mx(const Operands& o, const uint8_t* W, const float* x, float* y,
   const int want = std::max(1, std::min((nb + 63) / 64, 512 / groups));
   const int per_slice = (nb + want - 1) / want;
   const int slices = (nb + per_slice - 1) / per_slice;
-  const int xwgs = groups * slices;
+  const int xwgs = encode_x ? groups * slices : 0;
   const long long items = static_cast<long long>((n + 31) / 32) * ((k / 64 + 7) / 8);
-  const int wwgs = static_cast<int>((items + 7) / 8);
-  mx_prep<<<static_cast<unsigned>(xwgs) + wwgs + (p.ks == 2 ? 512 : 0), 512, 0, s>>>(
-      x, m, k, slices, per_slice, xwgs, o.xf, o.xr, o.xflag, o.xspread, o.rexp, W, n, o.wf, wwgs, y, ldy);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  const int wwgs = encode_w ? static_cast<int>((items + 7) / 8) : 0;
+  const int clear = p.ks == 2 ? 512 : 0;
+  if (xwgs + wwgs + clear > 0) {
+    mx_prep<<<static_cast<unsigned>(xwgs) + wwgs + clear, 512, 0, s>>>(
+        x, m, k, slices, per_slice, xwgs, o.xf, o.xr, o.xflag, o.xspread, o.rexp, W, n, o.wf, wwgs, y, ldy);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   switch (p.tile) {
     case 0: return launch_tile<4, 2, 2, 4, 4>(o, y, W, x, m, n, ldy, k, p, s);
     case 1: return launch_tile<2, 2, 2, 4, 6>(o, y, W, x, m, n, ldy, k, p, s);
     default: return launch_tile<2, 2, 2, 2, 4>(o, y, W, x, m, n, ldy, k, p, s);
   }
+}
+
+// Chunks of at most `most` (at least 256) as even as multiples of 256 allow.
+int even_chunk(int count, long long most) {
+  const int cap = static_cast<int>(std::max<long long>(256, std::min<long long>(most / 256 * 256, INT_MAX / 2)));
+  const int chunks = (count + cap - 1) / cap;
+  return ((count + chunks - 1) / chunks + 255) / 256 * 256;
 }
 
 }  // namespace
@@ -644,12 +655,10 @@ hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n
                            hipStream_t s, StreamWorkspace* ws) {
   const auto* w = static_cast<const uint8_t*>(W);
   const int nb = k / 32;
-  // Activation rows in chunks whose digits (twice 3.25 bytes an element) take at
-  // most 256 MB, weight rows in chunks of at most 256 MB (0.875 bytes a weight).
-  const long long fit = (256LL << 20) / (7LL * k) / 256 * 256;
-  const int mchunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, INT_MAX / 2)));
-  const long long nfit = (256LL << 20) / k / 256 * 256;
-  const int nchunk = static_cast<int>(std::max<long long>(256, std::min<long long>(nfit, INT_MAX / 2)));
+  // Activation rows in chunks whose digits (3.25 bytes an element) take at most
+  // 256 MB, and as much for their further digits; weight rows in chunks of at most 256 MB (0.875 bytes a weight).
+  const int mchunk = even_chunk(m, (256LL << 20) / (4LL * k));
+  const int nchunk = even_chunk(n, (256LL << 20) / k);
   const size_t mpad = (std::min(m, mchunk) + 255) / 256 * 256;   // read in whole tiles
   const size_t xf_bytes = mpad / 32 * nb * kXBlock, flag_bytes = mpad / 8 * (nb + 1);
   const size_t wf_bytes = static_cast<size_t>((std::min(n, nchunk) + 31) / 32) * nb * kWBlock + 128;   // kWSlot reads
@@ -665,9 +674,11 @@ hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n
   e = stream_buffer(ws, s, sizeof(int) * mpad, 1, &buf);
   if (e != hipSuccess) return e;
   o.rexp = static_cast<int*>(buf);
-  for (int m0 = 0; m0 < m; m0 += mchunk)
-    for (int n0 = 0; n0 < n; n0 += nchunk) {
-      e = run_mx(o, w + static_cast<long long>(n0) * nb * 18,
+  // each chunk of weights encoded once, its rows inside; the rows once where
+  // they are one chunk
+  for (int n0 = 0; n0 < n; n0 += nchunk)
+    for (int m0 = 0; m0 < m; m0 += mchunk) {
+      e = run_mx(o, m > mchunk || n0 == 0, m0 == 0, w + static_cast<long long>(n0) * nb * 18,
                  x + static_cast<long long>(m0) * k, y + static_cast<long long>(m0) * n + n0,
                  std::min(mchunk, m - m0), std::min(nchunk, n - n0), n, k, s);
       if (e != hipSuccess) return e;

@@ -795,3 +795,27 @@ def test_cint8_f16_route_codes_near_zero_points(qc, dev, m, rows, cols, gsize, s
     y64 = x.double() @ wd.T.contiguous()
     err = (y.double() - y64).norm(dim=0) / y64.norm(dim=0)
     assert float(err.max()) < 2e-6, float(err.max())
+
+
+@pytest.mark.parametrize("m,storage", [(4700, 0), (9300, 1)])
+def test_cint8_f16_route_chunks(qc, dev, m, storage):
+    """More rows than the 256 MB of activation fragments hold at once (f32 and
+    f16), with zero points that leave something."""
+    import torch
+    rows, cols, groups = 130, 14336, 112
+    print(f"cint8 f16 chunks m={m} storage={storage}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m)
+    codes = torch.randint(-128, 128, (rows, cols), generator=g, device=dev, dtype=torch.int8)
+    scales = 1e-3 * (0.5 + torch.rand((rows, groups), generator=g, device=dev))
+    z = 40.0 * torch.randn((rows, groups), generator=g, device=dev)
+    w = qc.cint8_weights(codes, scales, z, rows, cols, groups)
+    wd = ((codes.double().reshape(rows, groups, -1) - z.double()[:, :, None]) *
+          scales.double()[:, :, None]).reshape(rows, cols)
+    x = torch.randn((m, cols), generator=g, device=dev)
+    x = x if storage == 0 else x.half()
+    y = torch.full((m, rows), float("nan"), device=dev)
+    assert qc.cint8_project_raw(0, [w], x, storage, m, [y], [0]) == 0
+    torch.cuda.synchronize()
+    y64 = x.double() @ wd.T.contiguous()
+    err = (y.double() - y64).norm(dim=1) / y64.norm(dim=1)
+    assert float(err.max()) < 2e-6, float(err.max())

@@ -220,3 +220,40 @@ def test_q4_digits_outliers(qc, oracle, dev, kind, m, n, k):
         assert float(new.norm() / size.norm()) <= float(old.norm() / size.norm()) + 3e-7
         # row by row, a row's own draw of roundings aside
         assert bool((new <= 1.5 * old + 3e-7 * size).all()), float((new / old).max())
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [
+    (1, 4700, 2079, 14336),     # 6-bit form: two chunks of rows, the first in two K ranges
+    (1, 400, 18945, 14336),     # two chunks of columns
+    (1, 4700, 18945, 14336),    # both
+    (1, 4700, 300, 14336), (0, 4700, 300, 14336)])   # f16 form: two chunks of rows
+def test_chunks(qc, dev, fmt, m, n, k):
+    """Calls whose encoded operands pass the 256 MB of a chunk, with ragged
+    remainders in both directions, rows that the 6-bit form gives further
+    digits and one that is not finite in each chunk of rows."""
+    import torch
+    print(f"chunks fmt={fmt} m={m} n={n} k={k}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    P = qc.pack(fmt, torch.randn((n, k), generator=g, device=dev) * 0.02)
+    x = torch.randn((m, k), generator=g, device=dev)
+    x[::50, 77] = 3000.0
+    bad = [7, m - 3]
+    x[bad, 1234] = float("nan")
+    y, z = (torch.full((m, n), float("nan"), device=dev) for _ in range(2))
+    for out in (y, z):
+        assert qc.qgemm_raw(fmt, P, x, out, m, n, k) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int32), z.view(torch.int32))
+    assert bool(torch.isnan(y[bad]).all())
+    del z
+    w = qc.unpack(fmt, P, n, k).double()
+    x[bad] = 0.0
+    y[bad] = 0.0
+    wt = w.T.contiguous()
+    for r in range(0, m, 1024):
+        xs = x[r:r + 1024].double()
+        y64 = xs @ wt
+        err = (y[r:r + 1024].double() - y64).abs()
+        assert bool((err <= TOL * xs.norm(dim=1, keepdim=True) * w.norm(dim=1)[None, :]).all()), r
+        rel = float(err.norm() / y64.norm())
+        assert rel < 2e-6, (r, rel)
