@@ -137,7 +137,7 @@ hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, i
 
 // The q4_0 form of it that re-encodes weights and activations for the
 // block-scaled 6-bit MFMA, and the sizes it is taken for.
-bool mx_pays(int m, int n);
+bool mx_pays(int m, int n, int k);
 hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n, int k,
                            hipStream_t s, StreamWorkspace* ws);
 

@@ -644,12 +644,21 @@ int even_chunk(int count, long long most) {
 
 }  // namespace
 
-// Re-encoding the weights pays from about 384 rows: N = 14336, K = 4096, M =
-// 256 / 384 / 512: f16 form 84 / 123 / 134 us, this one 80 / 97 / 106; N =
-// 4096: M = 384 / 512 / 1024 47 / 58 / 89 against 46 / 53 / 72.  Narrow matrices
-// leave its larger tiles too few workgroups (M = 384, N = 1000, K = 1024: 15.5
-// against 20.1 us).
-bool mx_pays(int m, int n) { return m >= 384 && n >= 2048; }
+// The 6-bit form saves about a quarter of the f16 form's time where it fills
+// the chip, against about 8 us of encoding and of a second prep's latency (so
+// from 4.8e9 products), and its larger tiles leave CUs idle below some 2.3e6
+// outputs, more with long K, which the f16 form cuts into up to eight ranges.
+// Measured over 280 shapes, f16 / 6-bit form in us: K = 512 N = 6144 M = 768 24.5
+// / 23.5, N = 14336 M = 512 / 2048 26.0 / 28.3 and 79.3 / 70.4; K = 1024 N = 4096
+// M = 512 / 1024 / 2048 20.1 / 27.0, 30.9 / 31.2 and 47.1 / 42.1; K = 4096 N = 2048
+// M = 384 / 1024 / 2048 34.8 / 41.8, 54.2 / 56.0 and 92.9 / 79.1, N = 4096 M = 512 /
+// 768 49.8 / 51.1 and 75.1 / 66.2, N = 14336 M = 384 / 512 118 / 88 and 123 / 101;
+// K = 14336 N = 2048 M = 512 / 2048 90 / 132 and 290 / 251, N = 4096 M = 512 / 1024
+// 143 / 151 and 250 / 236.  The worst pick is 5% off the faster form.
+bool mx_pays(int m, int n, int k) {
+  const double outs = static_cast<double>(m) * n;
+  return m >= 384 && n >= 2048 && outs * k >= 4.8e9 && outs >= 2.3e6 + 40.0 * std::max(0, k - 4096);
+}
 
 hipError_t launch_qgemm_mx(const void* W, const float* x, float* y, int m, int n, int k,
                            hipStream_t s, StreamWorkspace* ws) {

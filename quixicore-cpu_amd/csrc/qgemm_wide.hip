@@ -564,7 +564,7 @@ hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, in
 hipError_t launch_qgemm_wide(int fmt, const void* W, const float* x, float* y, int m, int n, int k,
                              int ranges, hipStream_t s, Scratch& scratch) {
   const auto* w = static_cast<const uint8_t*>(W);
-  if (fmt == kQ4_0 && ranges == 0 && mx_pays(m, n)) return launch_qgemm_mx(W, x, y, m, n, k, s, scratch.w);
+  if (fmt == kQ4_0 && ranges == 0 && mx_pays(m, n, k)) return launch_qgemm_mx(W, x, y, m, n, k, s, scratch.w);
   // Rows in chunks whose fragments (4 bytes an element) take at most 256 MB.
   const long long fit = (256LL << 20) / (4LL * k) / 256 * 256;
   const int chunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, INT_MAX / 2)));

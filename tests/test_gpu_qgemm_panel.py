@@ -98,15 +98,17 @@ def test_panel_prefill_sizes(qc, oracle, dev, fmt, m, n, k):
 
 # Automatic route: 33 rows (q4_0: 17) are the first 2-D call, and shapes around the edges
 # of its tiles (32 / 64 / 128 / 256 rows by 128 / 256 columns), with K of one block
-# pair, odd pairs, and K splits; from 384 rows and 2048 columns q4_0 takes the
-# re-encoded 6-bit form.
+# pair, odd pairs, and K splits; the last six take the re-encoded 6-bit form for
+# q4_0 (its three tiles, one and two K ranges).
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("m,n,k", [(17, 129, 64), (18, 127, 320), (31, 1361, 1088),
                                    (32, 4096, 4096), (32, 14337, 512),
                                    (33, 129, 64), (64, 2048, 4096), (65, 127, 320),
                                    (77, 1361, 1088), (257, 300, 448), (383, 2049, 192),
                                    (384, 2048, 64), (385, 2079, 576), (641, 2305, 128),
-                                   (1025, 4097, 192), (2049, 2080, 64)])
+                                   (1025, 4097, 192), (2049, 2080, 64),
+                                   (2049, 36900, 64), (1025, 24580, 192), (513, 14340, 1088),
+                                   (641, 6201, 2112), (385, 6201, 4160), (1025, 2305, 2112)])
 def test_wide_tile_edges(qc, oracle, dev, fmt, m, n, k):
     import torch
     print(f"wide fmt={fmt} m={m} n={n} k={k}", flush=True)
@@ -131,7 +133,8 @@ def test_wide_tile_edges(qc, oracle, dev, fmt, m, n, k):
     assert rel < (4e-6 if fmt == 1 and m >= 384 and n >= 2048 else 1e-6), rel
 
 
-@pytest.mark.parametrize("m,n,k", [(400, 2050, 320), (700, 4100, 64)])
+@pytest.mark.parametrize("m,n,k", [(400, 2050, 320), (700, 4100, 64), (385, 14340, 1088),
+                                   (2100, 36000, 64)])
 def test_q4_digits_range_and_nonfinite_rows(qc, oracle, dev, m, n, k):
     """The re-encoded q4_0 form with activations over 40 decades, zero,
     subnormal and huge rows, a misaligned x, and rows holding NaN or +-inf:
@@ -174,7 +177,7 @@ def test_q4_digits_range_and_nonfinite_rows(qc, oracle, dev, m, n, k):
         assert bool((y[r][inf].double() == want[inf]).all()), r
 
 
-@pytest.mark.parametrize("m,n,k", [(384, 2048, 1024), (400, 14340, 192), (770, 14340, 320)])
+@pytest.mark.parametrize("m,n,k", [(1025, 2305, 2112), (385, 6201, 4160), (513, 14340, 1088)])
 @pytest.mark.parametrize("kind", ["channels 50", "channels 100", "channels 1e4", "channels 1e6",
                                   "rows 1e3", "every block 1e3", "elements 50", "misaligned 1e3"])
 def test_q4_digits_outliers(qc, oracle, dev, kind, m, n, k):
@@ -182,7 +185,7 @@ def test_q4_digits_outliers(qc, oracle, dev, kind, m, n, k):
     zero or not: the re-encoded q4_0 form is no further from 64 bits than a
     hi + lo pair of bf16 activations (2^-18 of each element) would be, up to the
     2^-20 of the largest that eight digits are for.  (f32 sums add at most sqrt(K / 32) 2^-25 of the
-    result on either: 3e-7 covers it.)  Sizes for its three tiles, with one and
+    result on either: 4e-7 covers it.)  Sizes for its three tiles, with one and
     two K ranges."""
     import torch
     print(f"q4 outliers {kind} m={m} n={n} k={k}", flush=True)
@@ -217,9 +220,9 @@ def test_q4_digits_outliers(qc, oracle, dev, kind, m, n, k):
         old = (pair @ wt - y64).norm(dim=1)
         new = (y[:, half].double() - y64).norm(dim=1)
         size = y64.norm(dim=1)
-        assert float(new.norm() / size.norm()) <= float(old.norm() / size.norm()) + 3e-7
+        assert float(new.norm() / size.norm()) <= float(old.norm() / size.norm()) + 4e-7
         # row by row, a row's own draw of roundings aside
-        assert bool((new <= 1.5 * old + 3e-7 * size).all()), float((new / old).max())
+        assert bool((new <= 1.5 * old + 4e-7 * size).all()), float((new / old).max())
 
 
 @pytest.mark.parametrize("fmt,m,n,k", [
