@@ -156,7 +156,7 @@ inline TilePlan plan_tiles(const Tile* tiles, int count, int m, int n, int units
   for (int i = 0; i < count; ++i) {
     const Tile& c = tiles[i];
     const double wgs = static_cast<double>((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
-    for (int want : {1, 2, 3, 4, 6, 8}) {
+    for (int want : {1, 2, 3, 4, 6, 8, 12, 16, 24}) {
       if (ranges > 0 ? want != std::min(ranges, units) : want > max_ks) continue;
       const int per = (units + want - 1) / want;
       const int ks = (units + per - 1) / per;

@@ -490,7 +490,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void wide_gemm(
 // K = 14336: 98 us for 16 workgroups, 111 for 224): a workgroup more than there
 // are CUs costs a round (two share a CU's operand feed), and its ring is nine
 // steps deep, because a step is only one MFMA tile (N = 14336, K = 4096, two K
-// ranges: 25.7 us with seven steps, 24.4 with nine, 25.5 with fifteen).
+// ranges: 25.7 us with seven steps, 24.4 with nine, 25.5 with fifteen).  It may
+// take up to 24 K ranges: with few columns and long K eight leave most CUs
+// idle (M = 17, K = 14336, N = 64 / 256 / 2048 23.2 / 23.6 / 24.9 us with eight,
+// 18.7 / 19.3 / 21.5 with more; bf16 passes 19.5 / 20.5 / 24.4).
 constexpr int kTiles = 4;   // for more than 32 rows
 constexpr Tile kTile[kTiles + 1] = {{256, 256, 1, 2.84, 4.10},
                                 {128, 256, 1, 1.70, 2.30},
@@ -519,7 +522,7 @@ hipError_t run_wide(const uint8_t* W, const float* x, float* y, int m, int n, in
                                            : static_cast<double>(scratch.fixed_bytes) -
                                                  static_cast<double>(scratch.fixed_split + xf_bytes);
   const int cus = device_cu_count();
-  TilePlan p = m <= 32 ? plan_tiles(&kTile[kTiles], 1, m, n, k / 64, cus, ranges, 8, left)
+  TilePlan p = m <= 32 ? plan_tiles(&kTile[kTiles], 1, m, n, k / 64, cus, ranges, 24, left)
                        : plan_tiles(kTile, kTiles, m, n, k / 64, cus, ranges, 8, left);
   if (m <= 32) p.tile = kTiles;
   const long long outs = static_cast<long long>(m) * n;

@@ -101,7 +101,8 @@ def test_panel_prefill_sizes(qc, oracle, dev, fmt, m, n, k):
 # pair, odd pairs, and K splits; the last six take the re-encoded 6-bit form for
 # q4_0 (its three tiles, one and two K ranges).
 @pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("m,n,k", [(17, 129, 64), (18, 127, 320), (31, 1361, 1088),
+@pytest.mark.parametrize("m,n,k", [(17, 64, 14336), (25, 333, 8256), (32, 1000, 16448),
+                                   (17, 129, 64), (18, 127, 320), (31, 1361, 1088),
                                    (32, 4096, 4096), (32, 14337, 512),
                                    (33, 129, 64), (64, 2048, 4096), (65, 127, 320),
                                    (77, 1361, 1088), (257, 300, 448), (383, 2049, 192),
