@@ -136,9 +136,15 @@ __global__ __launch_bounds__(512) void f16_prep(const void* __restrict__ x, int 
     *reinterpret_cast<f16x8*>(d) = hi;
     if constexpr (P == 2) *reinterpret_cast<f16x8*>(d + kSlotBytes) = lo;
     if (sums > 0) {
-      sum += __shfl_xor(sum, 8);
-      sum += __shfl_xor(sum, 32);
-      if (sums == 1) sum += __shfl_xor(sum, 16);
+      sum += dpp_f32<0x128>(sum);                  // lane ^ 8 (a rotation of 16 lanes)
+      const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum),
+                                                      false, false);
+      sum = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+      if (sums == 1) {
+        const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum),
+                                                        false, false);
+        sum = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+      }
       if (lane < 16 * sums && s == 0)
         xs[(static_cast<long long>(m >> 5) * steps * sums + t * sums + (sums == 2 ? b : 0)) * 32 +
            (m & 31)] = sum;
@@ -167,7 +173,7 @@ __device__ __forceinline__ T* pick(T* a, T* b, bool second) {
 
 // The part of a zero point that codes can be reduced by exactly in f16.
 __device__ __forceinline__ float code_zero(float z) {
-  return fminf(fmaxf(rintf(z), -1152.0f), 896.0f);
+  return __builtin_amdgcn_fmed3f(rintf(z), -1152.0f, 896.0f);
 }
 
 // The projection of activation row xr (elements) on weight row n in the

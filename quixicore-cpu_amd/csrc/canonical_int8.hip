@@ -870,8 +870,12 @@ hipError_t launch_cint8(const CInt8Launch& L, hipStream_t s) {
   // 64 x 256 output tiles fill at most half of the CUs: N = 4096 M = 256 60 /
   // 37 and 47, M = 512 63 / 41 and 54; N = 14336 M = 256 67 / 70 and 95.  (Every
   // rule is the same for f32 and 16-bit activations, whose results have the
-  // same bits.)  Lengths the planes do not take go here as well.
-  const long long plane_tiles = (m + 63LL) / 64 * ((L.w[0].rows * (L.mode == 1 ? 2 : 1) + 255) / 256);
+  // same bits.)  Of several matrices the tallest decides, in any order, as in a call of
+  // its own (row scales, M = 1024, heights 1024, 4096 and 4096: 196 / 166 and 233).
+  // Lengths the planes do not take go here as well.
+  long long tallest = 0;
+  for (int i = 0; i < L.nw; ++i) tallest = std::max<long long>(tallest, L.w[i].rows);
+  const long long plane_tiles = (m + 63LL) / 64 * ((tallest * (L.mode == 1 ? 2 : 1) + 255) / 256);
   const bool planes_fit = k <= kPlanesMaxK && (!grp || k % 128 == 0);
   const bool f16_pays = !grp ? m > 128 && 2 * plane_tiles <= device_cu_count()
                         : sg.gsize == 32 ? m > (aff ? 32 : 64)

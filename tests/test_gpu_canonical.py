@@ -819,3 +819,24 @@ def test_cint8_f16_route_chunks(qc, dev, m, storage):
     y64 = x.double() @ wd.T.contiguous()
     err = (y.double() - y64).norm(dim=1) / y64.norm(dim=1)
     assert float(err.max()) < 2e-6, float(err.max())
+
+
+def test_cint8_route_of_several_matrices(qc, dev):
+    """Matrices of very different heights over one x: the route does not depend
+    on which of them comes first, so each output has the same bits in any order."""
+    import torch
+    m, cols = 1024, 256
+    print("cint8 heights", flush=True)
+    g = torch.Generator(device=dev).manual_seed(11)
+    mats = []
+    for rows in (64, 16384, 300):
+        c = torch.randint(-127, 128, (rows, cols), generator=g, device=dev, dtype=torch.int8)
+        s = 1e-2 * (0.5 + torch.rand((rows, 1), generator=g, device=dev))
+        mats.append((c, s, qc.cint8_weights(c, s, None, rows, cols, 1)))
+    x = torch.randn((m, cols), generator=g, device=dev)
+    outs = {}
+    for order in ((0, 1, 2), (1, 0, 2), (2, 1, 0)):
+        ys = [torch.empty((m, mats[i][0].shape[0]), device=dev) for i in order]
+        assert qc.cint8_project_raw(0, [mats[i][2] for i in order], x, 0, m, ys, [0, 0, 0]) == 0
+        for i, y in zip(order, ys):
+            assert torch.equal(outs.setdefault(i, y).view(torch.int32), y.view(torch.int32)), order
