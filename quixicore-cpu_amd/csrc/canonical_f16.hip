@@ -563,27 +563,47 @@ size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
 }  // namespace
 
-hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k, hipStream_t s) {
-  const int p = L.xtype == QC_STORAGE_F32 ? 2 : 1;
-  const int nmat = L.mode == 1 ? 1 : L.nw;
-  const int gps = sg.groups == 1 ? 0 : sg.gsize == 32 ? 2 : 1;
-  const size_t es = p == 2 ? 4 : 2;
-  const bool vec = reinterpret_cast<uintptr_t>(L.x) % 16 == 0 && L.ldx % (16 / es) == 0;
-  // rows in chunks whose fragments take at most 256 MB
-  const long long fit = (256LL << 20) / (2LL * p * k) / 256 * 256;
-  const int chunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, 1 << 20)));
-  const int rows = std::min(chunk, (m + 255) / 256 * 256);
-  std::unique_lock<std::mutex> hold;
-  uint8_t* base = nullptr;
-  const size_t xf_bytes = up256(2ull * p * rows * k);
-  // zero points: the rows' sums over 32 (groups of 32) or 64 columns
+namespace {
+
+// A call's scratch: the fragments of `rows` activation rows (chunks of at most
+// 256 MB), their exponents, and with zero points their sums over 32 (groups of
+// 32) or 64 columns.
+struct F16Scratch {
+  int p, gps, sums, chunk, rows;
+  size_t xf_bytes, bytes;
+};
+F16Scratch f16_scratch(const CSegs& sg, const CInt8Launch& L, int m, int k) {
+  F16Scratch f;
+  f.p = L.xtype == QC_STORAGE_F32 ? 2 : 1;
+  f.gps = sg.groups == 1 ? 0 : sg.gsize == 32 ? 2 : 1;
   bool zeros = false;
   for (int i = 0; i < L.nw; ++i) zeros = zeros || sg.zero[i] != nullptr;
-  const int sums = !zeros ? 0 : gps == 2 ? 2 : 1;
-  hipError_t e = call_scratch(s, xf_bytes + 4ull * rows + 4ull * rows * (k / 64) * sums, hold,
-                              reinterpret_cast<void**>(&base));
+  f.sums = !zeros ? 0 : f.gps == 2 ? 2 : 1;
+  const long long fit = (256LL << 20) / (2LL * f.p * k) / 256 * 256;
+  f.chunk = static_cast<int>(std::max<long long>(256, std::min<long long>(fit, 1 << 20)));
+  f.rows = std::min(f.chunk, (m + 255) / 256 * 256);
+  f.xf_bytes = up256(2ull * f.p * f.rows * k);
+  f.bytes = f.xf_bytes + 4ull * f.rows + 4ull * f.rows * (k / 64) * f.sums;
+  return f;
+}
+
+}  // namespace
+
+size_t cint8_f16_scratch(const CSegs& sg, const CInt8Launch& L, int m, int k) {
+  return f16_scratch(sg, L, m, k).bytes;
+}
+
+hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k, hipStream_t s) {
+  const F16Scratch f = f16_scratch(sg, L, m, k);
+  const int p = f.p, gps = f.gps, sums = f.sums, chunk = f.chunk, rows = f.rows;
+  const int nmat = L.mode == 1 ? 1 : L.nw;
+  const size_t es = p == 2 ? 4 : 2;
+  const bool vec = reinterpret_cast<uintptr_t>(L.x) % 16 == 0 && L.ldx % (16 / es) == 0;
+  std::unique_lock<std::mutex> hold;
+  uint8_t* base = nullptr;
+  hipError_t e = call_scratch(s, f.bytes, hold, reinterpret_cast<void**>(&base));
   if (e != hipSuccess) return e;
-  int* rexp = reinterpret_cast<int*>(base + xf_bytes);
+  int* rexp = reinterpret_cast<int*>(base + f.xf_bytes);
   float* xs = reinterpret_cast<float*>(rexp + rows);
   for (int m0 = 0; m0 < m; m0 += chunk) {
     const int mc = std::min(chunk, m - m0);

@@ -816,6 +816,16 @@ hipError_t call_scratch(hipStream_t s, size_t bytes, std::unique_lock<std::mutex
   return stream_buffer(ws, s, bytes, 0, out);
 }
 
+bool call_scratch_ready(hipStream_t s, size_t bytes) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  StreamWorkspace* ws = nullptr;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap == hipStreamCaptureStatusNone ||
+      stream_workspace(s, &ws) != hipSuccess)
+    return true;
+  std::lock_guard<std::mutex> hold(ws->call);
+  return ws->bytes[0] >= bytes;
+}
+
 // Host entry (all checks done by the caller): see CInt8Launch in qc_internal.h.
 hipError_t launch_cint8(const CInt8Launch& L, hipStream_t s) {
   CSegs sg{};
@@ -881,8 +891,11 @@ hipError_t launch_cint8(const CInt8Launch& L, hipStream_t s) {
                         : sg.gsize == 32 ? m > (aff ? 32 : 64)
                         : sg.gsize == 64 ? m > 64
                                          : m > 64 && (aff || plane_tiles > device_cu_count());
+  // (Those lengths' other kernels, the digit dots below, take no scratch: a first
+  // such call within a capture stays on them.)
   if (fast && L.dot == 0 && L.mode != 2 && k % 64 == 0 &&
-      (!grp || sg.gsize == 32 || sg.gsize % 64 == 0) && (f16_pays || (!planes_fit && m > 32)))
+      (!grp || sg.gsize == 32 || sg.gsize % 64 == 0) && (f16_pays || (!planes_fit && m > 32)) &&
+      (planes_fit || call_scratch_ready(s, cint8_f16_scratch(sg, L, m, k))))
     return launch_cint8_f16(sg, L, m, k, s);
   // Two or more activation rows with row scales, three or more with scale
   // groups of 64 or a multiple of 128 columns, five or more with groups of

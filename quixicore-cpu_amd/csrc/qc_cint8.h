@@ -60,11 +60,15 @@ hipError_t launch_cint8_planes(const CSegs& sg, const CInt8Launch& L, int m, int
 // the caller: 16-byte aligned codes, K % 64 == 0, not the RoPE mode; groups of
 // 32 or a multiple of 64 columns.
 hipError_t launch_cint8_f16(const CSegs& sg, const CInt8Launch& L, int m, int k, hipStream_t s);
+size_t cint8_f16_scratch(const CSegs& sg, const CInt8Launch& L, int m, int k);   // its scratch bytes
 
 // The call's scratch: buffer 0 of its stream's cache entry, whose call lock
 // `hold` keeps until the caller's last launch.
 hipError_t call_scratch(hipStream_t s, size_t bytes, std::unique_lock<std::mutex>& hold,
                         void** out);
+// Whether that call can be served: false while s is capturing and the buffer
+// held is smaller, as it would then have to be allocated within the capture.
+bool call_scratch_ready(hipStream_t s, size_t bytes);
 
 namespace {   // device helpers: one copy per file
 

@@ -840,3 +840,48 @@ def test_cint8_route_of_several_matrices(qc, dev):
         assert qc.cint8_project_raw(0, [mats[i][2] for i in order], x, 0, m, ys, [0, 0, 0]) == 0
         for i, y in zip(order, ys):
             assert torch.equal(outs.setdefault(i, y).view(torch.int32), y.view(torch.int32)), order
+
+
+@pytest.mark.parametrize("m,rows,cols,gsize", [(40, 96, 16448, 0), (70, 130, 192, 64)])
+def test_cint8_first_call_within_a_capture(qc, dev, m, rows, cols, gsize):
+    """Lengths that the row planes do not take need no scratch in a capture: a
+    first call on a stream is captured without allocating, replays (with eager
+    calls on the same stream between them) give the captured call's result, and a
+    capture after an eager call, which leaves scratch, gives the eager bits."""
+    import torch
+    print(f"cint8 capture m={m} rows={rows} cols={cols} gsize={gsize}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m + cols)
+    groups = cols // gsize if gsize else 1
+    codes = torch.randint(-128, 128, (rows, cols), generator=g, device=dev, dtype=torch.int8)
+    scales = 1e-3 * (0.5 + torch.rand((rows, groups), generator=g, device=dev))
+    w = qc.cint8_weights(codes, scales, None, rows, cols, groups)
+    wd = (codes.double().reshape(rows, groups, -1) * scales.double()[:, :, None]).reshape(rows, cols)
+    x = torch.randn((m, cols), generator=g, device=dev)
+    y = torch.zeros((m, rows), device=dev)
+    eager = torch.zeros((m, rows), device=dev)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+
+    def call(out):
+        return qc.cint8_project_raw(0, [w], x, 0, m, [out], [0], stream=stream.cuda_stream)
+
+    bound = TOL * x.double().norm(dim=1, keepdim=True) * wd.norm(dim=1)[None, :]
+    y64 = x.double() @ wd.T.contiguous()
+    for warm in (False, True):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            assert call(y) == 0
+        first = None
+        for _ in range(3):
+            y.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bool(((y.double() - y64).abs() <= bound).all())
+            first = y.clone() if first is None else first
+            assert torch.equal(y.view(torch.int32), first.view(torch.int32))
+            assert call(eager) == 0
+            torch.cuda.synchronize()
+            assert bool(((eager.double() - y64).abs() <= bound).all())
+        if warm:
+            assert torch.equal(y.view(torch.int32), eager.view(torch.int32))
