@@ -516,14 +516,25 @@ hipError_t launch_int8_gemm(const int8_t* W, const int8_t* X, const float* ws, c
                                               asymmetric, status, s);
       // Fewer workgroups than that: a K step is then mostly latency (barrier,
       // LDS reads, loads), so the smallest tile that runs in one round, with
-      // two waves per SIMD for the larger of the two.  K = 4096, N = 4096,
-      // against 64 x 128 with four waves: M = 64 / 128 14.0 / 14.2 -> 9.7 / 10.0
-      // us (64 x 64), M = 301 16.1 -> 14.8, M = 512 17.4 -> 17.1 (128 x 64).
+      // two waves per SIMD for the larger of the two, and 128 x 128 where none
+      // does (LDS holds one workgroup of either a CU).  us, K = 4096 / 14336, 64
+      // x 128 with four waves, 64 x 64, 128 x 64, 128 x 128: N = 4096, M = 128 13.8 /
+      // 35.6, 9.8 / 24.9, 13.0 / 35.1, 18.0 / 47.4; M = 301 14.9 / 38.9, 15.4 / 43.4,
+      // 15.1 / 37.0, 18.9 / 47.9; M = 513 28.3 / 74.0, 23.5 / 67.3, 27.4 / 78.0, 20.9
+      // / 54.8.  With nearly every CU taken the four waves are the faster
+      // on long rows: M = 512 16.3 / 45.0, 17.6 / 52.1, 16.6 / 46.5 (K = 1024 8.4,
+      // 7.5, 7.4), N = 2048, M = 1000 16.2 / 44.3 against 16.7 / 47.1.
       if (tiles(64, 64) <= cus)
         return launch_ring<64, 64, 4, 2, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
                                             asymmetric, status, s);
-      return launch_ring<128, 64, 4, 4, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
-                                           asymmetric, status, s);
+      if (k >= 4096 && tiles(64, 128) <= cus && 5 * tiles(128, 64) > 4 * cus)
+        return launch_ring<64, 128, 4, 2, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
+                                             asymmetric, status, s);
+      if (tiles(128, 64) <= cus)
+        return launch_ring<128, 64, 4, 4, 2>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
+                                             asymmetric, status, s);
+      return launch_ring<128, 128, 4, 2, 4>(W, X, ws, as, row_sum, zp, y, acc_out, m, n, k,
+                                            asymmetric, status, s);
     }
     case kInt8Dma:
       if (wide)

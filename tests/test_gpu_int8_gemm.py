@@ -214,10 +214,11 @@ def test_validation_and_nonfinite_scales(qc, dev):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 64, 32), (63, 65, 96), (64, 4096, 4096), (129, 4033, 1056),
-                                   (301, 4096, 4128), (520, 3999, 160)])
+                                   (301, 4096, 4128), (520, 3999, 160), (500, 4033, 4128),
+                                   (513, 4001, 224), (1000, 2047, 4096)])
 def test_small_ring_tiles(qc, dev, m, n, k):
     """The automatic route's tiles for few workgroups (64 x 64 while they run
-    in one round, then 128 x 64), at their edges: exact accumulators, and the
+    in one round, then 128 x 64 or, on long rows, 64 x 128, then 128 x 128), at their edges: exact accumulators, and the
     epilogue's bits from them."""
     import torch
     print(f"int8 small tiles m={m} n={n} k={k}", flush=True)
