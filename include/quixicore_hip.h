@@ -384,7 +384,7 @@ int qc_hip_set_qgemm_rows(int mode);
  * at small N); everything else on
  * the kernels with exact int8 digit dots per 32-element block (the GEMV's
  * encoding of x) where they apply (K % 64 == 0, codes 16-byte aligned, row
- * scales or groups of >= 32 columns); 1 = never the row-plane route; -1 =
+ * scales or groups of >= 32 columns); 1 = neither MFMA route; -1 =
  * always the f32 multiply-add kernel.  All stay within the contract
  * tolerance.  Tuning and test knob with no reference counterpart. */
 int qc_hip_set_cint8_dot(int mode);

@@ -6,12 +6,13 @@
 // Numerics.  Activation rows are scaled by a power of two so that their
 // largest element lies in [2^14, 2^15).  f16 and bf16 activations are then f16
 // values (exactly, down to 2^-28 of the row's largest), f32 ones a pair hi + lo
-// of them within 2^-22 of each element.  Codes minus the integer of [-1152, 896]
+// of them within 2^-22 of each element plus 2^-25.  Codes minus the integer of [-1152, 896]
 // next to their zero point (at most 1280 in magnitude) are exact in f16,
 // products and sums are f32.  What of the zero point that leaves (up to 0.5 of a
 // fractional one) times the sum of x is subtracted in f32, so nothing is summed
-// that is larger than the codes' distances from their zero point.  An f32 row holding 16-bit values has lo = 0 throughout and gives the
-// bits of the 16-bit call.
+// that is larger than the codes' distances from their zero point.  An f32 row
+// holding 16-bit values has lo = 0 throughout and gives the bits of the 16-bit
+// call.
 //
 // What bounds it: with few workgroups the chain of a step (one barrier, the
 // LDS reads' latency, eight MFMAs: about 0.4 us per 64 columns); with a full

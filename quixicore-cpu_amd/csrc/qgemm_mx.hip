@@ -433,9 +433,6 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void mx_gemm(
     return groups >= 4 ? f : groups <= 0 ? 0u : f & ((1u << (8 * groups)) - 1);
   };
   uint32_t further = 0;
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
-    further |= in_rows(tm, reinterpret_cast<const uint32_t*>(xspread)[mt0 + wm * TM + tm]);
 
   if (steps > 0) {
     // Barrier B_s stands before the last m-tile of step s.  Step s issues,
@@ -447,6 +444,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void mx_gemm(
       for (int l = 0; l < C::G; ++l) issue(r, l);
       advance();
     }
+    typedef uint32_t Words __attribute__((ext_vector_type(TM)));   // (while those are in flight)
+    const Words spread = *reinterpret_cast<const Words*>(xspread + 4 * (mt0 + wm * TM));
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) further |= in_rows(tm, spread[tm]);
     wait_vmcnt<(S - 2) * C::G>();
     ring_barrier();
     i32x8 a[2][2], w[2][TN];                       // two buffers each
