@@ -100,8 +100,10 @@ __device__ __forceinline__ void byte_codes(uint32_t c, uint32_t& lo, uint32_t& h
 // One launch prepares both operands.  Workgroups [0, xwgs): eight activation
 // rows each and one of `slices` slices of K: the rows' power-of-two scales
 // (largest element in [0.5, 1)) and spreads, then the digits of the slice's
-// blocks, one lane per row and block.  The next wwgs: weights, a wave per n-tile and eight
-// block pairs, one lane per row and pair.  Any beyond clear y.
+// blocks, one lane per row and block.  The next wwgs: weights, a wave per n-tile
+// and two block pairs, one lane per row and pair (with eight pairs a wave the
+// last workgroups run on after the others: 14336 x 4096, M = 512 104 -> 99 us for
+// the whole call).  Any beyond clear y.
 __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int M, int K,
                                                int slices, int blocks_per_slice, int xwgs,
                                                uint8_t* __restrict__ xf, uint8_t* __restrict__ xr,
@@ -119,43 +121,41 @@ __global__ __launch_bounds__(512) void mx_prep(const float* __restrict__ x, int 
     return;
   }
   if (static_cast<int>(blockIdx.x) >= xwgs) {
-    const int groups = (npairs + 7) / 8;
+    const int groups = (npairs + 1) / 2;
     const int ntiles = (N + 31) / 32;
     const long long item = static_cast<long long>(blockIdx.x - xwgs) * 8 + wave;
-    const int nt = static_cast<int>(item / groups), g = static_cast<int>(item % groups);
-    if (nt >= ntiles) return;
+    const int nt = static_cast<int>(item / groups);
+    const int p = 2 * static_cast<int>(item % groups) + (lane >> 5);
+    if (nt >= ntiles || p >= npairs) return;
     const int col = lane & 31;
     const long long r = min(32 * nt + col, N - 1);
     const uint8_t* src = W + r * npairs * 36;
     uint8_t* dst = wf + static_cast<long long>(nt) * nb * kWBlock;
-    const int end = min(8 * g + 8, npairs);
-    for (int p = 8 * g + (lane >> 5); p < end; p += 2) {
-      const uint32_t* s = reinterpret_cast<const uint32_t*>(src + 36LL * p);
-      uint32_t q[9];
+    const uint32_t* s = reinterpret_cast<const uint32_t*>(src + 36LL * p);
+    uint32_t q[9];
 #pragma unroll
-      for (int i = 0; i < 9; ++i) q[i] = s[i];
+    for (int i = 0; i < 9; ++i) q[i] = s[i];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        uint32_t c[4];
+    for (int h = 0; h < 2; ++h) {
+      uint32_t c[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          c[i] = h == 0 ? __builtin_amdgcn_alignbyte(q[i + 1], q[i], 2) : q[5 + i];
-        uint32_t o[6];
+      for (int i = 0; i < 4; ++i)
+        c[i] = h == 0 ? __builtin_amdgcn_alignbyte(q[i + 1], q[i], 2) : q[5 + i];
+      uint32_t o[6];
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) {           // two dwords: 96 bits
-          uint32_t a, b, e, f;
-          byte_codes(c[i], a, b);
-          byte_codes(c[i + 1], e, f);
-          o[3 * (i / 2)] = a | (b << 24);
-          o[3 * (i / 2) + 1] = (b >> 8) | (e << 16);
-          o[3 * (i / 2) + 2] = (e >> 16) | (f << 8);
-        }
-        uint8_t* t = dst + static_cast<long long>(2 * p + h) * kWBlock;
-        *reinterpret_cast<u32x4*>(t + 16 * col) = u32x4{o[0], o[1], o[2], o[3]};
-        *reinterpret_cast<u32x2*>(t + 512 + 8 * col) = u32x2{o[4], o[5]};
-        *reinterpret_cast<float*>(t + 768 + 4 * col) =
-            half_bits_to_float(h == 0 ? q[0] & 0xFFFFu : q[4] >> 16);
+      for (int i = 0; i < 4; i += 2) {           // two dwords: 96 bits
+        uint32_t a, b, e, f;
+        byte_codes(c[i], a, b);
+        byte_codes(c[i + 1], e, f);
+        o[3 * (i / 2)] = a | (b << 24);
+        o[3 * (i / 2) + 1] = (b >> 8) | (e << 16);
+        o[3 * (i / 2) + 2] = (e >> 16) | (f << 8);
       }
+      uint8_t* t = dst + static_cast<long long>(2 * p + h) * kWBlock;
+      *reinterpret_cast<u32x4*>(t + 16 * col) = u32x4{o[0], o[1], o[2], o[3]};
+      *reinterpret_cast<u32x2*>(t + 512 + 8 * col) = u32x2{o[4], o[5]};
+      *reinterpret_cast<float*>(t + 768 + 4 * col) =
+          half_bits_to_float(h == 0 ? q[0] & 0xFFFFu : q[4] >> 16);
     }
     return;
   }
@@ -620,7 +620,7 @@ hipError_t run_mx(const Operands& o, bool encode_x, bool encode_w, const uint8_t
   const int per_slice = (nb + want - 1) / want;
   const int slices = (nb + per_slice - 1) / per_slice;
   const int xwgs = encode_x ? groups * slices : 0;
-  const long long items = static_cast<long long>((n + 31) / 32) * ((k / 64 + 7) / 8);
+  const long long items = static_cast<long long>((n + 31) / 32) * ((k / 64 + 1) / 2);
   const int wwgs = encode_w ? static_cast<int>((items + 7) / 8) : 0;
   const int clear = p.ks == 2 ? 512 : 0;
   if (xwgs + wwgs + clear > 0) {
