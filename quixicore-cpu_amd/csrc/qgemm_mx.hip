@@ -33,11 +33,11 @@
 //
 // What bounds it: VALU issue and MFMA power (16 fold FMAs and two MFMAs of 32
 // cycles per tile and block).  Weights are re-encoded once per call (0.875
-// bytes a weight, 18 us for 14336 x 4096, in the launch that encodes the
+// bytes a weight, most of 20 us for 14336 x 4096, in the launch that encodes the
 // activations), which decoding in the GEMM would repeat for every 128 or 256
-// rows of x.  q4_0, N = 14336, K = 4096: M = 512 139 -> 106 us, M = 2048
-// 552 -> 330 us (with blocks of eight digits: a third of them 125 and 444 us,
-// all 210 and 713).
+// rows of x.  q4_0, N = 14336, K = 4096: M = 512 139 -> 102 us, M = 2048
+// 552 -> 328 us (with blocks of eight digits: a third of them 116 and 440 us,
+// all 205 and 713).
 #include <algorithm>
 #include <climits>
 #include <type_traits>
